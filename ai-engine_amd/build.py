@@ -32,6 +32,7 @@ SOURCES = [
     "pkv_kvcopy.hip",
     "pkv_decode.hip",
     "pkv_prefill.hip",
+    "pkv_prefill_split.hip",
     "pkv_mixed.hip",
     "pkv_rope.hip",
     "pkv_sample.hip",
@@ -52,6 +53,7 @@ COMMON = [
 # so does the mixed launch, which runs the same prefill body.
 EXTRA = {
     "pkv_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "pkv_prefill_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "pkv_mixed.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -147,12 +147,18 @@ hipError_t plaunch_r(int R, const PrefillKArgs& k, hipStream_t s) {
 
 template <int DT>
 hipError_t plaunch_hd(int HD, int R, const PrefillKArgs& k, hipStream_t s) {
+  if constexpr (DT == PKV_F32) {
+    if (HD == 64) return launch_prefill_split(k, s);
+  }
   switch (HD) {
-    case 64: return plaunch_r<DT, 64>(R, k, s);
+    case 64:
+      if constexpr (DT != PKV_F32) return plaunch_r<DT, 64>(R, k, s);
+      break;
     case 128: return plaunch_r<DT, 128>(R, k, s);
     case 256: return plaunch_r<DT, 256>(R, k, s);
-    default: return hipErrorInvalidValue;
+    default: break;
   }
+  return hipErrorInvalidValue;
 }
 
 template <int HD>
@@ -173,6 +179,11 @@ int ilog2p(int x) {
 // Keys per tile and rows per workgroup of the kernel instantiated for a
 // pool's dtype and head_dim (host mirror of PCfg).
 void prefill_shape(int dt, int hd, int* kt, int* rows) {
+  if (dt == PKV_F32 && hd == 64) {
+    *kt = kSplitKeys;
+    *rows = kSplitRows;
+    return;
+  }
   const int rbytes = hd * (dt == PKV_F32 ? 4 : 2);
   *kt = rbytes >= 512 ? 32 : (rbytes >= 256 ? 64 : PKV_PREFILL_KT);
   *rows = kPW * 16 * ((dt != PKV_F32 && hd <= 128) ? PKV_PREFILL_NR : 1);

@@ -111,6 +111,13 @@ struct PrefillKArgs {
 // (nothing when the launch does not split).
 PrefillKArgs prefill_kargs(const pkv_pool* p, int layer, const PrefillArgs& a, char* partials);
 hipError_t launch_prefill_merge(const pkv_pool* p, const PrefillKArgs& k, hipStream_t stream);
+// f32 pools of head_dim 64 (pkv_prefill_split.hip): rows per workgroup and
+// keys per step, and the launch.
+#ifndef PKV_SPLIT_ROWS
+#define PKV_SPLIT_ROWS 128
+#endif
+constexpr int kSplitRows = PKV_SPLIT_ROWS, kSplitKeys = 64;
+hipError_t launch_prefill_split(const PrefillKArgs& k, hipStream_t s);
 
 // Workgroups of the launch; sets the row-block count and the XCD affinity
 // mapping of k for the kernel instantiated as PCfg<DT, HD, RT>.
@@ -141,6 +148,76 @@ namespace {
 // block's last key.
 __device__ __forceinline__ int n_parts_of(int prior, int part_keys) {
   return 1 + prior / part_keys;
+}
+
+// Work item of workgroup bid: (sequence, kv head) pair sg, row block rb, key
+// part, and the sequence's q0 = cu_q_lens[s], q1 = cu_q_lens[s + 1], ctx =
+// context_lens[s]; false past the last item.
+__device__ __forceinline__ bool prefill_item(const PrefillKArgs& a, int bid, int& sg, int& rb,
+                                             int& part, int& q0, int& q1, int& ctx) {
+  // ---- work item: (sequence, kv head) pair sg, row block rb, key part ----
+  // Row blocks run last (longest) first, each with its parts in order.
+  const int n_sg = a.n_seqs * a.kvh;
+  const int rbp = a.row_blocks * a.max_parts;
+  bool have_lens = false;
+  {
+    int u;
+    if (a.per_xcd > 0) {
+      const int x = bid % kXcd;
+      int slot = bid / kXcd;
+      const int nx = (n_sg - x + kXcd - 1) / kXcd;  // pairs of this XCD
+      if (slot >= nx * rbp) return false;
+      if (nx <= 64) {
+        // Heaviest first, paired per CU.  The XCD's pairs are ranked by
+        // context length (the key count of their last row; ties by index)
+        // and their items taken pair-major, last row block first.  The
+        // XCD's workgroups fill its CUs in rounds of cpx (one per CU per
+        // round); every other full round runs in reverse, so a CU holding
+        // the k-th heaviest item of one round holds the k-th lightest of
+        // the next.  A CU's older workgroup issues first, and here it is
+        // the heavier one.
+        if (a.cpx > 0) {
+          const int round = slot / a.cpx;
+          if ((round & 1) && (round + 1) * a.cpx <= nx * rbp)
+            slot = round * a.cpx + (a.cpx - 1 - slot % a.cpx);
+        }
+        // lane j: the j-th pair of the XCD, with its sequence's lengths
+        const int ln = threadIdx.x & 63;
+        const int sj = ln < nx ? (x + kXcd * ln) / a.kvh : 0;
+        const int w = ln < nx ? a.context_lens[sj] : -1;
+        const int c0 = a.cu_q_lens[sj], c1 = a.cu_q_lens[sj + 1];
+        int rank = 0;
+        for (int j = 0; j < nx; ++j) {
+          const int wj = __builtin_amdgcn_readlane(w, j);
+          rank += (wj > w) | ((wj == w) & (j < ln));
+        }
+        const int want = slot / rbp;
+        const int jw = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(ln < nx && rank == want));
+        sg = x + kXcd * jw;
+        ctx = __builtin_amdgcn_readlane(w, jw);
+        q0 = __builtin_amdgcn_readlane(c0, jw);
+        q1 = __builtin_amdgcn_readlane(c1, jw);
+        have_lens = true;
+        u = slot % rbp;
+      } else {
+        u = slot / nx;
+        sg = x + kXcd * (slot % nx);
+      }
+    } else {
+      if (bid >= n_sg * rbp) return false;
+      u = bid / n_sg;
+      sg = bid % n_sg;
+    }
+    rb = a.row_blocks - 1 - u / a.max_parts;
+    part = u % a.max_parts;
+  }
+  if (!have_lens) {
+    const int s = sg / a.kvh;
+    q0 = a.cu_q_lens[s];
+    q1 = a.cu_q_lens[s + 1];
+    ctx = a.context_lens[s];
+  }
+  return true;
 }
 
 template <int DT>
@@ -181,6 +258,51 @@ constexpr int prefill_wave_keys() {
   return (DT == PKV_F32 ? 2 : 1) * kWave / PCfg<DT, HD, 1>::CH;
 }
 
+// Fused store of the K/V rows of the chunk's tokens at positions prior + i.
+// Row blocks partition the tokens: token j belongs to the row block of its
+// first row, j R / ROWS, so row block r owns tokens tok_lo(r) ..
+// tok_lo(r + 1) - 1 with tok_lo(r) = ceil(r ROWS / R).  The store's load
+// round trip must not lengthen the heaviest row blocks (the last ones,
+// which see the most keys): row block rb of the sequence's nrb stores its
+// own tokens and those of its mirror nrb - 1 - rb when rb is the lighter of
+// the two, nothing when it is the heavier; only the last part of a row
+// block stores.  No workgroup of this launch reads these rows from the
+// pool: keys >= prior come from k_new / v_new.  kh, vh, kin, vin: the pool's
+// and the new rows' K and V at this kv head; NT threads.
+template <int ROWS, int RB, int NT>
+__device__ __forceinline__ void prefill_store_chunk(const PrefillKArgs& a, int R, int rb, int n_rows,
+                                                    int q_len, int prior, int q0, bool last_part,
+                                                    const int32_t* table, const char* kh,
+                                                    const char* vh, const char* kin,
+                                                    const char* vin) {
+  constexpr int CH = RB / 16;
+  const int nrb = (n_rows + ROWS - 1) / ROWS;
+  const int mirror = nrb - 1 - rb;
+  if (!last_part || rb > mirror) return;
+  const int BS = 1 << a.bs_log2;
+  const size_t slot_stride = (size_t)a.kvh * RB;
+  const size_t blk_stride = (size_t)BS * slot_stride;
+  auto tok_lo = [&](int r) { return min((r * ROWS + R - 1) / R, q_len); };
+  const int own0 = tok_lo(rb), own = tok_lo(rb + 1) - own0;
+  const int mir0 = tok_lo(mirror), mir = rb < mirror ? tok_lo(mirror + 1) - mir0 : 0;
+  const int nch = (own + mir) * CH;
+  for (int idx = threadIdx.x; idx < nch; idx += NT) {
+    const int j = idx / CH, c16 = 16 * (idx % CH);
+    const int tok = j < own ? own0 + j : mir0 + (j - own);
+    const int pos = prior + tok;
+    const int blk = table[pos >> a.bs_log2];
+    if ((unsigned)blk >= (unsigned)a.num_blocks) {
+      atomicOr(a.err, PKV_EBIT_BLOCK);
+      continue;
+    }
+    const size_t off = (size_t)blk * blk_stride + (size_t)(pos & (BS - 1)) * slot_stride + c16;
+    const size_t src = (size_t)(q0 + tok) * slot_stride + c16;
+    const u32x4 kx = ld16(kin + src), vx = ld16(vin + src);
+    st16(const_cast<char*>(kh) + off, kx);
+    st16(const_cast<char*>(vh) + off, vx);
+  }
+}
+
 // RT: the GQA ratio the kernel is built for, or 0 for any ratio (a.rq); the
 // ratio only enters the row <-> (token, head) index arithmetic.
 // SB (block_size below prefill_wave_keys): a wave-load's keys span several
@@ -199,72 +321,11 @@ __device__ __forceinline__ void prefill_body(const PrefillKArgs& a, int bid,
   const int G = lane >> 4;
   const int col = lane & 15;
 
-  // ---- work item: (sequence, kv head) pair sg, row block rb, key part ----
-  // Row blocks run last (longest) first, each with its parts in order.
-  const int n_sg = a.n_seqs * a.kvh;
-  const int rbp = a.row_blocks * a.max_parts;
-  int sg, rb, part;
-  int q0 = 0, q1 = 0, ctx = 0;  // cu_q_lens[s], cu_q_lens[s + 1], context_lens[s]
-  bool have_lens = false;
-  {
-    int u;
-    if (a.per_xcd > 0) {
-      const int x = bid % kXcd;
-      int slot = bid / kXcd;
-      const int nx = (n_sg - x + kXcd - 1) / kXcd;  // pairs of this XCD
-      if (slot >= nx * rbp) return;
-      if (nx <= 64) {
-        // Heaviest first, paired per CU.  The XCD's pairs are ranked by
-        // context length (the key count of their last row; ties by index)
-        // and their items taken pair-major, last row block first.  The
-        // XCD's workgroups fill its CUs in rounds of cpx (one per CU per
-        // round); every other full round runs in reverse, so a CU holding
-        // the k-th heaviest item of one round holds the k-th lightest of
-        // the next.  A CU's older workgroup issues first, and here it is
-        // the heavier one.
-        if (a.cpx > 0) {
-          const int round = slot / a.cpx;
-          if ((round & 1) && (round + 1) * a.cpx <= nx * rbp)
-            slot = round * a.cpx + (a.cpx - 1 - slot % a.cpx);
-        }
-        // lane j: the j-th pair of the XCD, with its sequence's lengths
-        const int ln = threadIdx.x & 63;
-        const int sj = ln < nx ? (x + kXcd * ln) / a.kvh : 0;
-        const int w = ln < nx ? a.context_lens[sj] : -1;
-        const int c0 = a.cu_q_lens[sj], c1 = a.cu_q_lens[sj + 1];
-        int rank = 0;
-        for (int j = 0; j < nx; ++j) {
-          const int wj = __builtin_amdgcn_readlane(w, j);
-          rank += (wj > w) | ((wj == w) & (j < ln));
-        }
-        const int want = slot / rbp;
-        const int jw = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(ln < nx && rank == want));
-        sg = x + kXcd * jw;
-        ctx = __builtin_amdgcn_readlane(w, jw);
-        q0 = __builtin_amdgcn_readlane(c0, jw);
-        q1 = __builtin_amdgcn_readlane(c1, jw);
-        have_lens = true;
-        u = slot % rbp;
-      } else {
-        u = slot / nx;
-        sg = x + kXcd * (slot % nx);
-      }
-    } else {
-      if (bid >= n_sg * rbp) return;
-      u = bid / n_sg;
-      sg = bid % n_sg;
-    }
-    rb = a.row_blocks - 1 - u / a.max_parts;
-    part = u % a.max_parts;
-  }
+  int sg, rb, part, q0, q1, ctx;
+  if (!prefill_item(a, bid, sg, rb, part, q0, q1, ctx)) return;
   const int g = sg % a.kvh;
   const int s = sg / a.kvh;
 
-  if (!have_lens) {
-    q0 = a.cu_q_lens[s];
-    q1 = a.cu_q_lens[s + 1];
-    ctx = a.context_lens[s];
-  }
   const int q_len_raw = q1 - q0;
   const int q_len = min(q_len_raw, a.max_q_len);
   const bool reporter = tid == 0 && rb == 0 && g == 0;
@@ -291,41 +352,11 @@ __device__ __forceinline__ void prefill_body(const PrefillKArgs& a, int bid,
   const int nparts = n_parts_of(prior, a.part_keys);
   if (part >= nparts) return;  // uniform over the workgroup
 
-  // Fused store of the K/V rows of the chunk's tokens at positions prior + i.
-  // Row blocks partition the tokens: token j belongs to the row block of its
-  // first row, j R / ROWS, so row block r owns tokens tok_lo(r) ..
-  // tok_lo(r + 1) - 1 with tok_lo(r) = ceil(r ROWS / R).  The store's load
-  // round trip must not lengthen the heaviest row blocks (the last ones,
-  // which see the most keys): row block rb of the sequence's nrb stores its
-  // own tokens and those of its mirror nrb - 1 - rb when rb is the lighter of
-  // the two, nothing when it is the heavier; only the last part of a row
-  // block stores.  No workgroup of this launch reads these rows from the
-  // pool: keys >= prior come from k_new / v_new.
   const char* kin = FUSED ? a.k_new + (size_t)g * C::RB : nullptr;
   const char* vin = FUSED ? a.v_new + (size_t)g * C::RB : nullptr;
-  const int nrb = (n_rows + C::ROWS - 1) / C::ROWS;
-  const int mirror = nrb - 1 - rb;
-  if (FUSED && part == nparts - 1 && rb <= mirror) {
-    auto tok_lo = [&](int r) { return min((r * C::ROWS + R - 1) / R, q_len); };
-    const int own0 = tok_lo(rb), own = tok_lo(rb + 1) - own0;
-    const int mir0 = tok_lo(mirror), mir = rb < mirror ? tok_lo(mirror + 1) - mir0 : 0;
-    const int nch = (own + mir) * C::CH;
-    for (int idx = tid; idx < nch; idx += kPT) {
-      const int j = idx / C::CH, c16 = 16 * (idx % C::CH);
-      const int tok = j < own ? own0 + j : mir0 + (j - own);
-      const int pos = prior + tok;
-      const int blk = table[pos >> a.bs_log2];
-      if ((unsigned)blk >= (unsigned)a.num_blocks) {
-        atomicOr(a.err, PKV_EBIT_BLOCK);
-        continue;
-      }
-      const size_t off = (size_t)blk * blk_stride + (size_t)(pos & tmask) * slot_stride + c16;
-      const size_t src = (size_t)(q0 + tok) * a.kvh * C::RB + c16;
-      const u32x4 kx = ld16(kin + src), vx = ld16(vin + src);
-      st16(const_cast<char*>(kh) + off, kx);
-      st16(const_cast<char*>(vh) + off, vx);
-    }
-  }
+  if constexpr (FUSED)
+    prefill_store_chunk<C::ROWS, C::RB, kPT>(a, R, rb, n_rows, q_len, prior, q0, part == nparts - 1,
+                                             table, kh, vh, kin, vin);
   const int k_hi = part + 1 < nparts ? (part + 1) * a.part_keys : n_keys;
   const int t_lo = part * (a.part_keys / C::KT);
   const int n_tiles = (k_hi + C::KT - 1) / C::KT;  // tiles t_lo .. n_tiles - 1

@@ -301,3 +301,39 @@ def test_fused_store_matches_oracle(gpu):
     _close(got.cpu().numpy(), case.reference(), "fused store vs oracle")
     assert np.array_equal(case.cache.read_bytes(0, pagedkv.K), case.kp.view(np.uint8).reshape(-1))
     case.close()
+
+
+# f32 pools of head_dim 64 (three bf16 parts per value, two key groups of 32
+# keys per step, 128 rows per workgroup): rows and keys around those edges.
+# |gpu - ref| <= 4e-6 max|v|: a weight's relative error is that of its exponent
+# (below 2^-24 x 16 in the log2 domain for these scores, twice), its exp2 (1
+# ulp) and the dropped products (2^-24), 2.2e-6 in all, the sums' roundings
+# random and below 1e-6.
+@pytest.mark.parametrize("R", [1, 7, 8])
+@pytest.mark.parametrize("prior,chunk", [(0, 1), (0, 31), (0, 33), (0, 64), (31, 2), (32, 128),
+                                         (33, 129), (63, 65), (1100, 19), (2048, 1)])
+def test_f32_split_products(gpu, R, prior, chunk):
+    c = PCase(gpu, wl.F32, 2 * R, 2, 64, 16, [prior, 5], [chunk, 40], seed=prior + chunk + R)
+    err = np.abs(c.run() - c.reference())
+    assert err.max() <= 4e-6 * np.abs(c.vp).max(), err.max()
+    c.close()
+
+
+def test_f32_split_values_beyond_bf16(gpu):
+    # a value whose bf16 part overflows, and infinities: what f32 arithmetic
+    # gives, row by row, and the rows that do not see them stay as they were
+    c = PCase(gpu, wl.F32, 4, 2, 64, 16, [0, 20], [70, 60], seed=5)
+    blk = lambda s, pos: (c.tables[s, pos // 16], pos % 16)
+    b, o = blk(0, 40)
+    c.vp[b, o, 0, 3], c.vp[b, o, 0, 5] = 3.4e38, -np.inf
+    b, o = blk(1, 50)
+    c.kp[b, o, 1, 0], c.q[:, :, 0] = -np.inf, np.abs(c.q[:, :, 0]) + 0.1  # weight 0
+    c.cache.write_bytes(0, pagedkv.K, c.kp)
+    c.cache.write_bytes(0, pagedkv.V, c.vp)
+    got, ref = c.run(), c.reference()
+    kp, vp = c.kp.copy(), c.vp.copy()
+    fin = np.isfinite(ref)
+    assert not fin.all() and np.array_equal(got[~fin], ref[~fin])
+    scale = np.maximum(np.abs(ref[fin]), np.abs(vp[np.abs(vp) < 1e38]).max())
+    assert (np.abs(got[fin] - ref[fin]) <= 4e-6 * scale).all()
+    c.close()
