@@ -566,3 +566,19 @@ def test_decode_positions_refuses_null(gpu):
                                           None, 64, 2, 32, c.scale, None, None, None)
     assert rc == pagedkv._lib.PKV_ERR_INVALID
     c.close()
+
+
+@pytest.mark.parametrize("hd,R,dt,out", [(64, 4, wl.F16, torch.float16), (64, 7, wl.F32, None),
+                                         (128, 8, wl.BF16, torch.bfloat16), (128, 1, wl.BF16, None),
+                                         (256, 3, wl.F16, torch.float16)])
+@pytest.mark.parametrize("longest", [2048, 2049, 2111, 4500])
+def test_merge_of_many_partitions(gpu, hd, R, dt, out, longest):
+    # 64-token partitions (a small batch): 32 is the last count merged by one
+    # wave per head, 33 the first by a workgroup per head; sequences of one
+    # partition, of none to merge, and of every remainder of a round beside it
+    c = Case(gpu, dt, 2 * R, 2, hd, 16, [longest - 1, 0, 63, 64, 1000], seed=hd + R)
+    ref = c.reference()[0]
+    got = c.run(out_dtype=out)
+    tol = {wl.F32: 0.0, wl.F16: 2.0 ** -11, wl.BF16: 2.0 ** -8}[dt] if out else 0.0
+    assert (np.abs(got - ref) <= ATOL + (RTOL + tol) * np.abs(ref)).all()
+    c.close()
