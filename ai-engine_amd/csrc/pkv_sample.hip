@@ -1479,10 +1479,14 @@ struct ExactArgs {
 // Which kernel selected a row's token (pkv_sample_exact_routes).
 constexpr int32_t kRouteArgmax = 0, kRouteBuckets = 1, kRouteRuns = 2, kRouteSort = 3;
 
+struct ExactLds {
+  SampleSmem sm;
+  ExactSmem xs;
+};
 template <int DT, bool VEC>
-__global__ void __launch_bounds__(kST) sample_exact_kernel(ExactArgs a) {
-  __shared__ SampleSmem sm;
-  __shared__ ExactSmem xs;
+__device__ __forceinline__ void exact_row(const ExactArgs& a, ExactLds& u) {
+  SampleSmem& sm = u.sm;
+  ExactSmem& xs = u.xs;
   const int row = a.row0 + blockIdx.x;
   const int tid = threadIdx.x;
   if (a.fallback && a.fallback[row] == 0) return;  // selected by an earlier kernel
@@ -1855,13 +1859,12 @@ __device__ __forceinline__ void f32_runs(RunSmem& rs, const RunArrays& ra, int R
 // sample_exact_kernel for 16-bit logits, on runs instead of a sorted copy.
 // Scratch: 4 kMaxRuns words per row (keys, counts, starts, values).
 template <int DT, bool VEC>
-__global__ void __launch_bounds__(kST) sample_runs_kernel(ExactArgs a) {
+__device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
   // Keys are 16-bit: of the logits themselves, or for f32 logits of their
   // bf16 value, which is the logit itself when its low 16 bits are zero (f32
   // logits of a bf16 model); a row with any other f32 logit is left to
   // sample_exact_kernel (a.fallback).
   constexpr int KT = DT == PKV_F32 ? PKV_BF16 : DT;
-  __shared__ RunLds u;
   __shared__ unsigned int wtmp[kSW];
   SampleSmem& sm = u.x.sm;
   RunSmem& rs = u.x.rs;
@@ -2057,6 +2060,32 @@ __global__ void __launch_bounds__(kST) sample_runs_kernel(ExactArgs a) {
   }
 }
 
+template <int DT, bool VEC>
+__global__ void __launch_bounds__(kST) sample_runs_kernel(ExactArgs a) {
+  __shared__ RunLds u;
+  runs_row<DT, VEC>(a, u);
+}
+template <int DT, bool VEC>
+__global__ void __launch_bounds__(kST) sample_exact_kernel(ExactArgs a) {
+  __shared__ ExactLds u;
+  exact_row<DT, VEC>(a, u);
+}
+// f32 rows the buckets left: runs of equal values when every logit is a bf16
+// value, else the sort.  One launch: rows that are done (usually all) exit.
+union LeftLds {
+  RunLds r;
+  ExactLds e;
+};
+template <bool VEC>
+__global__ void __launch_bounds__(kST) sample_left_kernel(ExactArgs a) {
+  __shared__ LeftLds u;
+  const int row = a.row0 + blockIdx.x;
+  if (a.fallback[row] == 0) return;  // uniform: selected by the buckets
+  runs_row<PKV_F32, VEC>(a, u.r);
+  __syncthreads();
+  exact_row<PKV_F32, VEC>(a, u.e);  // (returns when the runs selected the token)
+}
+
 // ---- f32 logits: buckets of y instead of a sort -----------------------------
 // Only the f32 running sums depend on the sorted order, and only in part.
 // While a running sum stays inside one binade, each addition adds an integer
@@ -2122,6 +2151,8 @@ struct BucketSmem {
   float ch_sum[kRegionA / 64];    // chunks of 64 of the top: sums (estimates),
   int ch_e[kRegionA / 64];        //   the binade predicted at their start,
   int ch_d0[kRegionA / 64], ch_d1[kRegionA / 64];  // their deltas in it (even / odd start)
+  int grp_e[kBk / 64];            // groups of 64 buckets: the binade all were summed for,
+  unsigned int grp_d[kBk / 64];   //   and their increments' sum (at most kDeltaCap)
   unsigned long long exptab[32];   // kExp2Tab
   unsigned long long wu[kSW];
   unsigned int wtmp[kSW];
@@ -2239,16 +2270,17 @@ __device__ __forceinline__ void wave_sort_desc(uint32_t* keys, uint32_t* idx, in
   }
 }
 
-// Calls f(valid, i, x) for every logit x = row[i] with the whole wave
-// converged (lanes past the end get valid = false): 16-byte vectors, U in
-// flight, when VEC, then the elements past the last vector.
+// Calls f(valid, i, x) for every logit x = row[i], i in [lo, V) (lo a
+// multiple of 4), with the whole wave converged (lanes past the end get
+// valid = false): 16-byte vectors, U in flight, when VEC, then the elements
+// past the last vector.
 template <bool VEC, int U, class F>
-__device__ __forceinline__ void row_converged(const char* row, int V, F&& f) {
+__device__ __forceinline__ void range_converged(const char* row, int lo, int V, F&& f) {
   const int lane = threadIdx.x & 63, w0 = (threadIdx.x >> 6) * 64;
-  int done = 0;
+  int done = lo;
   if constexpr (VEC) {
     const int nvec = V / 4;
-    for (int base = w0; base < nvec; base += U * kST) {
+    for (int base = lo / 4 + w0; base < nvec; base += U * kST) {
       u32x4 wb[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -2355,6 +2387,30 @@ __device__ __forceinline__ void walk_top(const BucketSmem& bs, int hi, float& s,
 // tie, or the sum leaves its binade or reaches thr inside it.
 constexpr int kWhyRebin = 1, kWhyStore = 2;
 
+// Groups of 64 buckets (group g: buckets 64 g .. 64 g + 63) that the walk can
+// pass in one step: no stored bucket, no tie, all summed for one binade.
+constexpr int kGroupMixed = INT_MIN, kGroupEmpty = INT_MAX;
+__device__ __forceinline__ void bucket_groups(BucketSmem& bs) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int g = wv; g < kBk / 64; g += kSW) {
+    const int b = 64 * g + lane;
+    const bool some = bs.start[b + 1] > bs.start[b];
+    const unsigned long long iv = bs.inc[b];
+    const int e = bs.eg[b];
+    const unsigned long long full = __ballot(some);
+    const unsigned long long mixed =
+        __ballot((bs.flag[b] & kStored) != 0 || (some && ((iv >> 63) || e == kNoBinade)));
+    const int e0 = full ? readlane_i(e, __builtin_ctzll(full)) : 0;
+    const unsigned long long other = __ballot(some && e != e0);
+    const unsigned d = some ? (unsigned)min(iv, (unsigned long long)kDeltaCap) : 0u;
+    const unsigned sum = wave_incl_add_u32(d);  // 64 (2^24 + 1) < 2^32
+    if (lane == 63) {
+      bs.grp_e[g] = mixed | other ? kGroupMixed : full ? e0 : kGroupEmpty;
+      bs.grp_d[g] = min(sum, (unsigned)kDeltaCap);
+    }
+  }
+}
+
 // Wave 0: continues the walk from bucket bs.b with sum bs.s over buckets
 // [0, nbk) (`part` kept only below position len).  Stored buckets are walked
 // in sorted order; others are applied as prefix sums of their increments
@@ -2386,22 +2442,42 @@ __device__ __forceinline__ void walk_scan(BucketSmem& bs, const uint32_t* K, int
       b = e2;
       continue;
     }
+    const uint32_t sb = __float_as_uint(s);
+    const int sE = (int)((sb >> 23) & 255u);
+    const bool sn = sE >= 1 && sE <= 254 && !(sb >> 31);  // wave-uniform
+    const int es = sE - 127;
+    const long long n = (long long)((sb & 0x7fffffu) | 0x800000u);
+    if ((b & 63) == 0 && b + 64 <= nbk) {  // whole groups, one a lane
+      const int gg = (b >> 6) + lane;
+      const bool in = 64 * gg + 64 <= nbk;
+      const int ge = in ? bs.grp_e[gg] : kGroupMixed;
+      const unsigned long long okg = __ballot(ge == kGroupEmpty || (sn && ge == es));
+      const int run = ~okg ? __builtin_ctzll(~okg) : 64;
+      const long long nend =
+          n + (long long)wave_incl_add_u32(lane < run && ge != kGroupEmpty ? bs.grp_d[gg] : 0u);
+      const float send = nend < (1ll << 24) ? ldexpf((float)nend, es - 23) : INFINITY;
+      const unsigned long long stm =
+          __ballot(sn && lane < run && (nend >= (1ll << 24) || (use_thr && send >= thr)));
+      const int upto = stm ? __builtin_ctzll(stm) : run;
+      if (upto > 0) {
+        if (sn) s = readlane_f(send, upto - 1);
+        b += 64 * upto;
+        continue;
+      }
+    }
+    // bucket by bucket, to the end of its group
+    const int lim = min(64 - (b & 63), nbk - b);
     const int g = b + lane;
-    const bool have = g < nbk;
+    const bool have = lane < lim;
     const bool stored = have && (bs.flag[g] & kStored);
     const int e = have ? bs.eg[g] : kNoBinade;
     const unsigned c = have ? bs.start[g + 1] - bs.start[g] : 0u;
     const unsigned long long iv = have ? bs.inc[g] : 0ull;
     const unsigned d = (unsigned)min(iv, (unsigned long long)kDeltaCap);
-    const uint32_t sb = __float_as_uint(s);
-    const int sE = (int)((sb >> 23) & 255u);
-    const bool sn = sE >= 1 && sE <= 254 && !(sb >> 31);  // wave-uniform
-    const int es = sE - 127;
     // lanes 0 .. run-1: empty buckets, or buckets summed for this binade
     const unsigned long long okm =
         __ballot(have && !stored && (c == 0u || (sn && (iv >> 63) == 0ull && e == es)));
     const int run = ~okm ? __builtin_ctzll(~okm) : 64;
-    const long long n = (long long)((sb & 0x7fffffu) | 0x800000u);
     // 64 (2^24 + 1) < 2^32
     const long long nend = n + (long long)wave_incl_add_u32(lane < run && c ? d : 0u);
     const float send = nend < (1ll << 24) ? ldexpf((float)nend, es - 23) : INFINITY;
@@ -2415,7 +2491,7 @@ __device__ __forceinline__ void walk_scan(BucketSmem& bs, const uint32_t* K, int
       why = kWhyStore;
       break;
     }
-    if (b >= nbk || run == 64 || readlane_i(stored, run)) continue;
+    if (upto == lim || readlane_i(stored, run)) continue;
     todo = b;  // bucket b: summed for another binade, or a tie
     why = sn && readlane_i(e, run) != es ? kWhyRebin : kWhyStore;
     break;
@@ -2443,11 +2519,15 @@ struct BucketRow {
     return f < (float)kBk ? (int)f : kBk - 1;
   }
   template <class F>
-  __device__ __forceinline__ void each(F&& f) const {  // f(x', t) for every logit
-    for_each<PKV_F32, VEC, 4>(x, V, [&](int, float v) {
+  __device__ __forceinline__ void each_in(int lo, int hi, F&& f) const {  // f(x', t)
+    for_range<PKV_F32, VEC, 4>(x, lo, hi, [&](int, float v) {
       const float xp = neg ? -v : v;
       f(xp, xp / aT - ymax);
     });
+  }
+  template <class F>
+  __device__ __forceinline__ void each(F&& f) const {  // f(x', t) for every logit
+    each_in(0, V, static_cast<F&&>(f));
   }
 };
 
@@ -2460,16 +2540,24 @@ __device__ __forceinline__ bool sort_stored(BucketSmem& bs, uint32_t* K, uint32_
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (tid == 0) bs.big = 0;
   __syncthreads();
-  for (int b = b0 + wv; b < nbk; b += kSW) {
-    if ((bs.flag[b] & (kStored | kSorted)) != kStored) continue;  // wave-uniform
-    const int st = (int)bs.start[b], n = (int)bs.start[b + 1] - st;
-    if (n > kWaveSortMax) {
-      if (lane == 0) atomicAdd(&bs.big, 1);
-      continue;
+  // wave wv: buckets congruent to wv modulo kSW (neighbours, which are often
+  // stored together, go to different waves), 64 flags at a time
+  for (int i0 = 0; i0 < kBk / kSW; i0 += 64) {
+    const int bl = kSW * (i0 + lane) + wv;
+    unsigned long long todo = __ballot(bl >= b0 && bl < nbk &&
+                                       (bs.flag[bl] & (kStored | kSorted)) == kStored);
+    for (; todo; todo &= todo - 1) {
+      const int b = kSW * (i0 + __builtin_ctzll(todo)) + wv;
+      const int st = (int)bs.start[b], n = (int)bs.start[b + 1] - st;
+      if (n > kWaveSortMax) {
+        if (lane == 0) atomicAdd(&bs.big, 1);
+        continue;
+      }
+      wave_sort_desc(K + st, KI + st, n, bs.stage[wv]);
+      if (lane == 0) bs.flag[b] |= kSorted;
     }
-    wave_sort_desc(K + st, KI + st, n, bs.stage[wv]);
-    if (lane == 0) bs.flag[b] |= kSorted;
   }
+  static_assert(kBk / kSW % 64 == 0, "");
   __syncthreads();
   if (bs.big == 0) return true;
   uint32_t* stg = &bs.stage[0][0];
@@ -2531,8 +2619,7 @@ __device__ __forceinline__ bool bucket_walk(BucketSmem& bs, uint32_t* K, uint32_
   }
   __syncthreads();
   for (int c = wv; c < nch; c += kSW) {
-    float pre = 0.0f;
-    for (int q = 0; q < c; ++q) pre += bs.ch_sum[q];
+    const float pre = wsum_f32(lane < c ? bs.ch_sum[lane] : 0.0f);  // (nch <= 64)
     const int e = use_thr && pre > thr * 1.0625f ? kNoBinade : binade_of(pre);
     int d0 = 0, d1 = 0;
     if (e != kNoBinade) {  // wave-uniform
@@ -2554,8 +2641,9 @@ __device__ __forceinline__ bool bucket_walk(BucketSmem& bs, uint32_t* K, uint32_
     bs.s = 0.0f;
     bs.b = 0;
   }
-  __syncthreads();
   for (;;) {
+    bucket_groups(bs);
+    __syncthreads();
     if (wv == 0) walk_scan(bs, K, nA, bA, nbk, part, len, use_thr, thr, vf);
     __syncthreads();
     const int todo = bs.todo, why = bs.why;
@@ -2584,13 +2672,25 @@ __device__ __forceinline__ bool bucket_walk(BucketSmem& bs, uint32_t* K, uint32_
       __syncthreads();
       continue;
     }
-    // store the keys of todo and the next buckets not stored
+    // store the keys of todo and the next buckets not stored; x' outside the
+    // interval that maps to these buckets (widened by more than the roundings
+    // of y, t and the bucket) need no division
+    const int blast = min(nbk, todo + kGatherSpan) - 1;
+    float xlo = -INFINITY, xhi = INFINITY;
+    {
+      const double sc = (double)rw.scale, ym = (double)rw.ymax, at = (double)rw.aT;
+      const double dlo = todo / sc * (1.0 - 1e-6), dhi = (blast + 1) / sc * (1.0 + 1e-6);
+      const double ylo = ym - dhi - 1e-6 * (fabs(ym) + dhi), yhi = ym - dlo + 1e-6 * (fabs(ym) + dlo);
+      if (sc > 0.0 && blast < kBk - 1) xlo = (float)(ylo * at - 1e-6 * fabs(ylo * at));
+      if (sc > 0.0) xhi = (float)(yhi * at + 1e-6 * fabs(yhi * at));
+    }
     for (int b = todo + tid; b < min(nbk, todo + kGatherSpan); b += kST)
       if (!(bs.flag[b] & kStored)) bs.flag[b] = kGather;
     __syncthreads();
-    row_converged<VEC, 4>(rw.x, rw.V, [&](bool valid, int i, float v) {
+    for_each<PKV_F32, VEC, 8>(rw.x, rw.V, [&](int i, float v) {
       const float xp = rw.neg ? -v : v;
-      const int b = valid ? rw.bucket(xp / rw.aT - rw.ymax) : kBk;
+      if (!(xp >= xlo && xp <= xhi)) return;
+      const int b = rw.bucket(xp / rw.aT - rw.ymax);
       if (b < kBk && (bs.flag[b] & kGather)) {
         const unsigned p = bs.start[b] + atomicAdd(&bs.cur[b], 1u);
         K[p] = order_key(xp);
@@ -2607,38 +2707,82 @@ __device__ __forceinline__ bool bucket_walk(BucketSmem& bs, uint32_t* K, uint32_
   return true;
 }
 
-template <bool VEC>
-__global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
-  __shared__ BucketLds u;
-  SampleSmem& sm = u.sm;
-  BucketSmem& bs = u.bs;
-  const int row = a.row0 + blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const char* x = a.logits + (long long)row * a.stride_bytes;
-  const int V = a.vocab;
-  const float T = a.temps ? a.temps[row] : 0.0f;
-  if (T == 0.0f || V <= 1) {  // sample.rs:13-15
-    float bv;
-    int bi;
-    block_argmax<PKV_F32, VEC>(sm, x, 0, V, bv, bi);
-    if (tid == 0) {
-      a.tokens[row] = bi == INT_MAX ? 0 : bi;
-      a.fallback[row] = 0;
-      if (a.route) a.route[row] = kRouteArgmax;
-    }
-    return;
-  }
-  auto leave = [&]() {
-    if (tid == 0) a.fallback[row] = 1;
-  };
-  const bool neg = T < 0.0f;
-  const float aT = fabsf(T);  // y = x / T = x' / |T| with x' = x, or -x when T < 0
+// A row split over several workgroups (batches too small to fill the GPU with
+// one workgroup per row): the three passes over its logits run on G chunks
+// each, one launch per pass, and the steps between them and after them on
+// one workgroup per row, with the state in global memory in between.  Every
+// sum handed over is an integer (counts, fixed-point masses, unit
+// increments), so it does not depend on the chunks, and the token is the
+// same as with one workgroup.  Launches: extremes, mass, plan (prefixes and
+// predictions), store (keys and increments), finish (sorts, walks, token);
+// for 8 rows of 128,256 f32 logits 4.9, 10.3, 13.2, 14.6 and 33 to 54 us (one
+// more pass over a row that meets a tie) of kernel time, against 132 us for
+// the passes alone on one workgroup.
+struct BucketWs {  // per row
+  float hi[kMaxG], lo[kMaxG];  // per chunk: largest and smallest x'
+  int nan[kMaxG];
+  float gmax[kMaxG];           // greedy rows: the chunk's maximum,
+  int gidx[kMaxG];             //   and its index (INT_MAX: none)
+  unsigned int cnt[kBk + 1];
+  float pm[kBk + 1];
+  unsigned int start[kBk + 2];
+  unsigned long long mass[kBk];
+  unsigned long long inc[kBk];
+  unsigned int cur[kBk];
+  short eg[kBk];
+  unsigned char flag[kBk];
+  uint32_t topk[kRegionA], topi[kRegionA];
+  int left;                    // left to the later kernels (or greedy)
+};
 
-  // 1. the largest and smallest x', and whether a logit is NaN
-  if (tid < 32) bs.exptab[tid] = kExp2Tab[tid];
-  float hi = -INFINITY, lo = INFINITY;
+// Rows of fewer logits, or more rows, stay on one workgroup each: the five
+// launches cost about 20 us, the passes of a 32,000-logit row 33.  Calls, split
+// against one workgroup per row: 1 row of 128,256 93 against 170 us, 8 rows 94
+// against 165, 32 rows 132 against 190, 64 rows 179 against 218; with an earlier
+// form of both paths 2 rows of 32,000 98 against 91, 33 of 5,000 96 against 69
+// and 100 of 128,256 (two chunks each) 282 against 276.
+constexpr int kSplitMinVocab = 65536, kSplitMaxRows = 64;
+
+// Which part of a row's selection bucket_row does: all of it, or one of the
+// one-workgroup steps of a split row.
+constexpr int kRowWhole = 0, kRowPlan = 1, kRowFinish = 2;
+
+// kBk entries of a row's state, kPerT a thread: all loads before any use, so
+// that the arrays of a step arrive in one round trip.
+constexpr int kPerT = kBk / kST;
+template <typename T>
+__device__ __forceinline__ void take(const T* src, T (&r)[kPerT]) {
+#pragma unroll
+  for (int q = 0; q < kPerT; ++q) r[q] = src[threadIdx.x + q * kST];
+}
+template <typename T>
+__device__ __forceinline__ void put(T* dst, const T (&r)[kPerT]) {
+#pragma unroll
+  for (int q = 0; q < kPerT; ++q) dst[threadIdx.x + q * kST] = r[q];
+}
+
+// The row's extremes from its G chunks', one chunk a lane.
+__device__ __forceinline__ void chunk_extremes(const BucketWs& w, int G, float& hi, float& lo,
+                                               bool& nan) {
+  static_assert(kMaxG <= 64, "");
+  const int lane = threadIdx.x & 63;
+  hi = lane < G ? w.hi[lane] : -INFINITY;
+  lo = lane < G ? w.lo[lane] : INFINITY;
+  nan = __ballot(lane < G && w.nan[lane] != 0) != 0ull;
+  hi = wave_reduce32(hi, [](float p, float q) { return fmaxf(p, q); });
+  lo = wave_reduce32(lo, [](float p, float q) { return fminf(p, q); });
+}
+
+// 1. the largest and smallest x' of [lo, hi), and whether a logit is NaN
+// (every thread, after a barrier)
+template <bool VEC>
+__device__ __forceinline__ void bucket_extremes(BucketSmem& bs, const char* x, int lo_i, int hi_i,
+                                                bool neg, float& hi, float& lo, bool& anynan) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  hi = -INFINITY;
+  lo = INFINITY;
   bool nan = false;
-  for_each<PKV_F32, VEC, kRowBatch>(x, V, [&](int, float v) {
+  for_range<PKV_F32, VEC, kRowBatch>(x, lo_i, hi_i, [&](int, float v) {
     const float xp = neg ? -v : v;
     hi = fmaxf(hi, xp);
     lo = fminf(lo, xp);
@@ -2653,11 +2797,226 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
     bs.wi[wv] = wnan;
   }
   __syncthreads();
-  bool anynan = false;
+  anynan = false;
   for (int w = 0; w < kSW; ++w) {
     hi = fmaxf(hi, bs.wf[w]);
     lo = fminf(lo, bs.wg[w]);
     anynan |= bs.wi[w] != 0;
+  }
+}
+
+// 2. logits and approximate mass (2^-40 units) per bucket over [lo, hi); the
+// tail only counted.  cur and inc start at zero.
+template <bool VEC>
+__device__ __forceinline__ void bucket_mass(BucketSmem& bs, const BucketRow<VEC>& rw, int lo,
+                                            int hi) {
+  const int lane = threadIdx.x & 63;
+  rw.each_in(lo, hi, [&](float, float t) {
+    const int b = rw.bucket(t);
+    const unsigned long long tl = __ballot(b == kBk);
+    if (tl && lane == __builtin_ctzll(__ballot(true)))
+      atomicAdd(&bs.cur[kBk], (unsigned)__popcll(tl));
+    if (b < kBk) {
+      atomicAdd(&bs.cur[b], 1u);
+      atomicAdd(&bs.inc[b], (unsigned long long)(__expf(t) * 0x1p40f));
+    }
+  });
+}
+
+// 5. over [lo, hi): store the flagged buckets' keys and indices (the top in
+// topk / topi, the others in K / KI, at their bucket's cursor in cur); add up
+// the others' increments for the denominator, decided from __expf where it
+// settles the rounding (quick_inc) and otherwise from the exact value
+// (through a per-wave queue in LDS, so that the exact exponentials and splits
+// run on full waves).
+// QUEUE (cur in global memory): stored logits go through a per-wave queue in
+// the LDS of the top (not used by this pass then), so that a wave takes its
+// cursors 64 at a time instead of waiting for a few lanes' atomics after
+// every element.
+template <bool VEC, bool QUEUE>
+__device__ __forceinline__ void bucket_store(BucketSmem& bs, const BucketRow<VEC>& rw, int lo,
+                                             int hi, int nbk, int bA, unsigned int* cur,
+                                             uint32_t* topk, uint32_t* topi, uint32_t* K,
+                                             uint32_t* KI) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const BucketValue p_of{rw.aT, rw.ymax, 1.0f, 1.0f, 0, bs.exptab};
+  {
+    float* qt = reinterpret_cast<float*>(bs.stage[wv]);
+    int* qb = reinterpret_cast<int*>(bs.stage[wv]) + 128;
+    static_assert(kWaveSortMax >= 256, "a queue of 128 (t, bucket) pairs per wave");
+    int qn = 0;  // wave-uniform
+    auto emit = [&](int b, uint32_t key, uint32_t i) __attribute__((always_inline)) {
+      const unsigned p = bs.start[b] + atomicAdd(&cur[b], 1u);
+      if (b < bA) {
+        topk[p] = key;
+        topi[p] = i;
+      } else {
+        K[p] = key;
+        KI[p] = i;
+      }
+    };
+    constexpr int kQ = kRegionA / kSW;  // queue entries per wave
+    static_assert(kQ >= 128, "");
+    uint32_t* sk = bs.topk + wv * kQ;
+    uint32_t* si = bs.topi + wv * kQ;
+    int* sb = reinterpret_cast<int*>(bs.topv) + wv * kQ;
+    int sn = 0;  // wave-uniform
+    auto flush = [&](int n) __attribute__((always_inline)) {
+      if (lane < n) emit(sb[lane], sk[lane], si[lane]);
+    };
+    auto drain = [&](int n) {
+      if (lane < n) {
+        const int b = qb[lane];
+        add_inc(bs, b, p_of.of_t(qt[lane]), bs.eg[b]);
+      }
+    };
+    range_converged<VEC, 4>(rw.x, lo, hi, [&](bool valid, int i, float v) {
+      const float xp = rw.neg ? -v : v;
+      const float t = xp / rw.aT - rw.ymax;
+      const int b = valid ? rw.bucket(t) : kBk;
+      const bool play = b < nbk;
+      const unsigned char fl = play ? bs.flag[b] : 0;
+      const bool keep = play && (fl & kStored);  // the top, or another stored bucket
+      if constexpr (QUEUE) {
+        const unsigned long long m = __ballot(keep);
+        if (m) {  // wave-uniform
+          const int at = sn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+          if (keep) {
+            sb[at] = b;
+            sk[at] = order_key(xp);
+            si[at] = (uint32_t)i;
+          }
+          sn += __popcll(m);
+          if (sn >= 64) {
+            flush(64);
+            if (lane < sn - 64) {
+              sb[lane] = sb[64 + lane];
+              sk[lane] = sk[64 + lane];
+              si[lane] = si[64 + lane];
+            }
+            sn -= 64;
+          }
+        }
+      } else if (keep) {
+        emit(b, order_key(xp), (uint32_t)i);
+      }
+      const int e = play && !(fl & kStored) ? bs.eg[b] : kNoBinade;
+      bool push = false;
+      if (e != kNoBinade) {
+        unsigned qi;
+        if (!quick_inc(__expf(t), e, qi)) push = true;  // the exact value, through the queue
+        else if (qi) atomicAdd(&bs.inc[b], (unsigned long long)qi);
+      }
+      const unsigned long long m = __ballot(push);
+      if (m) {  // wave-uniform
+        const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (push) {
+          qt[at] = t;
+          qb[at] = b;
+        }
+        qn += __popcll(m);
+        if (qn >= 64) {
+          drain(64);
+          if (lane < qn - 64) {
+            qt[lane] = qt[64 + lane];
+            qb[lane] = qb[64 + lane];
+          }
+          qn -= 64;
+        }
+      }
+    });
+    drain(qn);
+    if constexpr (QUEUE) flush(sn);
+  }
+}
+
+// Positions [0, n) are kept: buckets [0, nbk) are in play and `part` (if >= 0)
+// is kept only in part (a cut inside the tail drops nothing that matters).
+__device__ __forceinline__ void bucket_cut(const BucketSmem& bs, int n, int& nbk, int& part) {
+  nbk = kBk;
+  part = -1;
+  if (n < (int)bs.start[kBk]) {  // the bucket of position n - 1: the last with start < n
+    int l = 0, h = kBk - 1;
+    while (l < h) {
+      const int mid = (l + h + 1) >> 1;
+      if ((int)bs.start[mid] < n) l = mid;
+      else h = mid - 1;
+    }
+    nbk = l + 1;
+    part = (int)bs.start[l + 1] > n ? l : -1;
+  }
+}
+
+// The top of the order: buckets [0, result), at most kRegionA positions (0:
+// bucket 0 alone holds more).
+__device__ __forceinline__ int bucket_top(const BucketSmem& bs, int nbk) {
+  int l = 0, h = nbk;
+  while (l < h) {
+    const int mid = (l + h + 1) >> 1;
+    if ((int)bs.start[mid] <= kRegionA) l = mid;
+    else h = mid - 1;
+  }
+  return l;
+}
+
+// The selection of one row (PART: kRowWhole) or its one-workgroup steps of a
+// split row (kRowPlan, kRowFinish; state in w, G chunks).
+template <bool VEC, int PART>
+__device__ __forceinline__ void bucket_row(const ExactArgs& a, BucketLds& u, BucketWs* w, int G) {
+  SampleSmem& sm = u.sm;
+  BucketSmem& bs = u.bs;
+  const int row = a.row0 + blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const char* x = a.logits + (long long)row * a.stride_bytes;
+  const int V = a.vocab;
+  const float T = a.temps ? a.temps[row] : 0.0f;
+  if (T == 0.0f || V <= 1) {  // sample.rs:13-15
+    if constexpr (PART == kRowFinish) return;
+    float bv;
+    int bi;
+    if constexpr (PART == kRowWhole) {
+      block_argmax<PKV_F32, VEC>(sm, x, 0, V, bv, bi);
+    } else {  // the chunks' maxima, in index order
+      bv = -INFINITY;
+      bi = INT_MAX;
+      const float gm = lane < G ? w->gmax[lane] : -INFINITY;
+      const int gi = lane < G ? w->gidx[lane] : INT_MAX;
+      for (int g = 0; g < G; ++g) {
+        const float v = readlane_f(gm, g);
+        if (v > bv) {
+          bv = v;
+          bi = readlane_i(gi, g);
+        }
+      }
+    }
+    if (tid == 0) {
+      a.tokens[row] = bi == INT_MAX ? 0 : bi;
+      a.fallback[row] = 0;
+      if (a.route) a.route[row] = kRouteArgmax;
+    }
+    return;
+  }
+  auto leave = [&]() {
+    if (tid == 0) {
+      a.fallback[row] = 1;
+      if constexpr (PART == kRowPlan) w->left = 1;
+    }
+  };
+  const bool neg = T < 0.0f;
+  const float aT = fabsf(T);  // y = x / T = x' / |T| with x' = x, or -x when T < 0
+
+  if (tid < 32) bs.exptab[tid] = kExp2Tab[tid];
+  if constexpr (PART == kRowFinish) {
+    if (w->left) return;  // uniform
+  }
+  float hi, lo;
+  bool anynan;
+  if constexpr (PART == kRowWhole) {
+    bucket_extremes<VEC>(bs, x, 0, V, neg, hi, lo, anynan);
+  } else {
+    chunk_extremes(*w, G, hi, lo, anynan);
   }
   const float ymax = hi / aT, ymin = lo / aT;
   if (anynan || !(fabsf(ymax) < INFINITY)) {  // uniform
@@ -2668,25 +3027,51 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
   const BucketRow<VEC> rw{x, V, neg, aT, ymax,
                           D > 0.0f ? fminf((float)kBk / D, 0x1p100f) : 0.0f};
 
-  // 2. logits and approximate mass (2^-40 units) per bucket; the tail only
-  // counted
-  for (int i = tid; i <= kBk; i += kST) bs.cur[i] = 0u;
-  for (int i = tid; i < kBk; i += kST) bs.inc[i] = 0ull;
-  __syncthreads();
-  rw.each([&](float, float t) {
-    const int b = rw.bucket(t);
-    const unsigned long long tl = __ballot(b == kBk);
-    if (tl && lane == __builtin_ctzll(__ballot(true)))
-      atomicAdd(&bs.cur[kBk], (unsigned)__popcll(tl));
-    if (b < kBk) {
-      atomicAdd(&bs.cur[b], 1u);
-      atomicAdd(&bs.inc[b], (unsigned long long)(__expf(t) * 0x1p40f));
-    }
-  });
-  __syncthreads();
+  // 2. counts and masses
+  if constexpr (PART == kRowWhole) {
+    for (int i = tid; i <= kBk; i += kST) bs.cur[i] = 0u;
+    for (int i = tid; i < kBk; i += kST) bs.inc[i] = 0ull;
+    __syncthreads();
+    bucket_mass<VEC>(bs, rw, 0, V);
+    __syncthreads();
+  } else if constexpr (PART == kRowPlan) {
+    unsigned c[kPerT];
+    unsigned long long m[kPerT];
+    take(w->cnt, c);
+    take(w->mass, m);
+    if (tid == 0) bs.cur[kBk] = w->cnt[kBk];
+    put(bs.cur, c);
+    put(bs.inc, m);
+    __syncthreads();
+  } else {  // the plan's state, and what the store pass added to it
+    unsigned st[kPerT], tk[kPerT], ti[kPerT];
+    float pmv[kPerT];
+    unsigned long long iv[kPerT];
+    short ev[kPerT];
+    unsigned char fv[kPerT];
+    take(w->start, st);
+    take(w->pm, pmv);
+    take(w->inc, iv);
+    take(w->eg, ev);
+    take(w->flag, fv);
+    take(w->topk, tk);
+    take(w->topi, ti);
+    if (tid < 2) bs.start[kBk + tid] = w->start[kBk + tid];
+    if (tid == 2) bs.pm[kBk] = w->pm[kBk];
+    put(bs.start, st);
+    put(bs.pm, pmv);
+    put(bs.inc, iv);
+    put(bs.eg, ev);
+    put(bs.flag, fv);
+    put(bs.topk, tk);
+    put(bs.topi, ti);
+    static_assert(kRegionA == kBk, "");
+    for (int i = tid; i <= kBk; i += kST) bs.cur[i] = 0u;
+    __syncthreads();
+  }
 
   // 3. exclusive prefixes: bucket starts (the tail last) and masses
-  {
+  if constexpr (PART != kRowFinish) {
     const int b0 = 4 * tid;
     unsigned c[4];
     unsigned long long m[4];
@@ -2751,42 +3136,21 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
   // top_k: positions [0, len) are kept; buckets [0, nbk) are in play and
   // `part` is kept only in part (a cut inside the tail drops nothing that
   // matters)
-  const int nreg = (int)bs.start[kBk];
   int len = a.top_k > 0 && a.top_k < V ? a.top_k : V;
   int nbk = kBk, part = -1;
-  auto cut_at = [&](int n) {
-    nbk = kBk;
-    part = -1;
-    if (n < nreg) {  // the bucket of position n - 1: the last with start < n
-      int l = 0, h = kBk - 1;
-      while (l < h) {
-        const int mid = (l + h + 1) >> 1;
-        if ((int)bs.start[mid] < n) l = mid;
-        else h = mid - 1;
-      }
-      nbk = l + 1;
-      part = (int)bs.start[l + 1] > n ? l : -1;
-    }
-  };
+  auto cut_at = [&](int n) { bucket_cut(bs, n, nbk, part); };
   cut_at(len);
   // the top of the order: buckets [0, bA), positions [0, nA), nA <= kRegionA
   // (bucket 0 must fit)
-  int bA = 0;
-  {
-    int l = 0, h = nbk;
-    while (l < h) {
-      const int mid = (l + h + 1) >> 1;
-      if ((int)bs.start[mid] <= kRegionA) l = mid;
-      else h = mid - 1;
-    }
-    bA = l;
-  }
+  const int bA = bucket_top(bs, nbk);
   if (bA == 0) {  // uniform: bucket 0 alone holds more than kRegionA logits
     leave();
     return;
   }
   const int nA = (int)bs.start[bA];
 
+  const bool has_p = a.top_p == a.top_p;  // Some(top_p)
+  if constexpr (PART != kRowFinish) {
   // 4. which buckets to store: the top, the top_k cut, the buckets around
   // each one where the denominator is predicted to leave its binade, and
   // (with a margin) each bucket where top_p's sum of p / S or r's of p / S
@@ -2803,7 +3167,6 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
   for (int q = 0; q < kBk / kST; ++q) egp[q] = binade_of(pc[tid + q * kST]);
   __syncthreads();  // (cur is cleared below)
   const float Sest = bs.pm[kBk];
-  const bool has_p = a.top_p == a.top_p;  // Some(top_p)
   const float S3est = Sest * (has_p ? fminf(fmaxf(a.top_p, 0x1p-20f), 1.0f) : 1.0f);
   auto reaches = [&](int b, float div, float thr) {
     return bs.pm[b] * (1.0f - kMargin) / div <= thr * (1.0f + kMargin) &&
@@ -2827,70 +3190,27 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
 #pragma unroll
   for (int q = 0; q < kBk / kST; ++q) bs.flag[tid + q * kST] = fl[q];
   __syncthreads();
+  }
+  if constexpr (PART == kRowPlan) {
+    for (int i = tid; i < kBk + 2; i += kST) w->start[i] = bs.start[i];
+    for (int i = tid; i <= kBk; i += kST) w->pm[i] = bs.pm[i];
+    for (int i = tid; i < kBk; i += kST) {
+      w->eg[i] = bs.eg[i];
+      w->flag[i] = bs.flag[i];
+      w->inc[i] = 0ull;
+      w->cur[i] = 0u;
+    }
+    if (tid == 0) w->left = 0;
+    return;
+  }
 
-  // 5. store the flagged buckets' keys (the top in LDS); the others'
-  // increments for the denominator, decided from __expf where it settles
-  // the rounding (quick_inc) and otherwise from the exact value (through a
-  // per-wave queue in LDS, so that the exact exponentials and splits run on
-  // full waves)
+  // 5. store the flagged buckets' keys (the top in LDS), add the others'
+  // increments
   uint32_t* K = a.scratch + (size_t)blockIdx.x * 2 * (size_t)V;  // keys
   uint32_t* KI = K + V;                                           // their indices
   const BucketValue p_of{aT, ymax, 1.0f, 1.0f, 0, bs.exptab};
-  {
-    float* qt = reinterpret_cast<float*>(bs.stage[wv]);
-    int* qb = reinterpret_cast<int*>(bs.stage[wv]) + 128;
-    static_assert(kWaveSortMax >= 256, "a queue of 128 (t, bucket) pairs per wave");
-    int qn = 0;  // wave-uniform
-    auto drain = [&](int n) {
-      if (lane < n) {
-        const int b = qb[lane];
-        add_inc(bs, b, p_of.of_t(qt[lane]), bs.eg[b]);
-      }
-    };
-    row_converged<VEC, 4>(x, V, [&](bool valid, int i, float v) {
-      const float xp = neg ? -v : v;
-      const float t = xp / aT - ymax;
-      const int b = valid ? rw.bucket(t) : kBk;
-      const bool play = b < nbk;
-      const unsigned char fl = play ? bs.flag[b] : 0;
-      if (play && (fl & kStored)) {  // the top in LDS, other stored buckets in K
-        const unsigned p = bs.start[b] + atomicAdd(&bs.cur[b], 1u);
-        if (b < bA) {
-          bs.topk[p] = order_key(xp);
-          bs.topi[p] = (uint32_t)i;
-        } else {
-          K[p] = order_key(xp);
-          KI[p] = (uint32_t)i;
-        }
-      }
-      const int e = play && !(fl & kStored) ? bs.eg[b] : kNoBinade;
-      bool push = false;
-      if (e != kNoBinade) {
-        unsigned qi;
-        if (!quick_inc(__expf(t), e, qi)) push = true;  // the exact value, through the queue
-        else if (qi) atomicAdd(&bs.inc[b], (unsigned long long)qi);
-      }
-      const unsigned long long m = __ballot(push);
-      if (m) {  // wave-uniform
-        const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        if (push) {
-          qt[at] = t;
-          qb[at] = b;
-        }
-        qn += __popcll(m);
-        if (qn >= 64) {
-          drain(64);
-          if (lane < qn - 64) {
-            qt[lane] = qt[64 + lane];
-            qb[lane] = qb[64 + lane];
-          }
-          qn -= 64;
-        }
-      }
-    });
-    drain(qn);
-  }
+  if constexpr (PART == kRowWhole)
+    bucket_store<VEC, false>(bs, rw, 0, V, nbk, bA, bs.cur, bs.topk, bs.topi, K, KI);
   __syncthreads();
   // the top, sorted in LDS: each key's rank within its bucket
   {
@@ -2911,12 +3231,7 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
     for (int q = 0; q < kRegionA / kST; ++q) {
       const int i = tid + q * kST;
       if (i >= nA) continue;
-      int l = 0, h = bA - 1;  // the bucket of position i: the last with start <= i
-      while (l < h) {
-        const int mid = (l + h + 1) >> 1;
-        if ((int)bs.start[mid] <= i) l = mid;
-        else h = mid - 1;
-      }
+      const int l = rw.bucket(key_value(mk[q]) / aT - ymax);  // its bucket
       const int st = (int)bs.start[l], en = (int)bs.start[l + 1];
       int r = 0;
       for (int j = st; j < en; ++j) {
@@ -3042,6 +3357,133 @@ __global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
   }
 }
 
+template <bool VEC>
+__global__ void __launch_bounds__(kST) sample_bucket_kernel(ExactArgs a) {
+  __shared__ BucketLds u;
+  bucket_row<VEC, kRowWhole>(a, u, nullptr, 0);
+}
+
+template <bool VEC, int PART>
+__global__ void __launch_bounds__(kST) bucket_step_kernel(ExactArgs a, BucketWs* ws, int G) {
+  __shared__ BucketLds u;
+  bucket_row<VEC, PART>(a, u, ws + blockIdx.x, G);
+}
+
+// Chunk blockIdx.x of row blockIdx.y: its extremes (greedy rows: its maximum);
+// also clears the row's counts and masses for the next launch.
+template <bool VEC>
+__global__ void __launch_bounds__(kST) bucket_extremes_kernel(ExactArgs a, BucketWs* ws) {
+  __shared__ BucketLds u;
+  const int row = a.row0 + blockIdx.y, g = blockIdx.x, G = gridDim.x, tid = threadIdx.x;
+  BucketWs& w = ws[blockIdx.y];
+  for (int i = g * kST + tid; i <= kBk; i += G * kST) w.cnt[i] = 0u;
+  for (int i = g * kST + tid; i < kBk; i += G * kST) w.mass[i] = 0ull;
+  const char* x = a.logits + (long long)row * a.stride_bytes;
+  const float T = a.temps[row];
+  int lo_i, hi_i;
+  split_chunk(a.vocab, lo_i, hi_i);
+  if (T == 0.0f) {
+    float bv;
+    int bi;
+    block_argmax<PKV_F32, VEC>(u.sm, x, lo_i, hi_i, bv, bi);
+    if (tid == 0) {
+      w.gmax[g] = bv;
+      w.gidx[g] = bi;
+    }
+    return;
+  }
+  float hi, lo;
+  bool nan;
+  bucket_extremes<VEC>(u.bs, x, lo_i, hi_i, T < 0.0f, hi, lo, nan);
+  if (tid == 0) {
+    w.hi[g] = hi;
+    w.lo[g] = lo;
+    w.nan[g] = nan;
+  }
+}
+
+// The row's buckets from its chunks' extremes; false for greedy rows and rows
+// the plan leaves to the later kernels.
+template <bool VEC>
+__device__ __forceinline__ bool split_row(const ExactArgs& a, const BucketWs& w, int row,
+                                          BucketRow<VEC>& rw) {
+  const float T = a.temps[row];
+  if (T == 0.0f) return false;
+  float hi, lo;
+  bool nan;
+  chunk_extremes(w, (int)gridDim.x, hi, lo, nan);
+  const float aT = fabsf(T), ymax = hi / aT, ymin = lo / aT;
+  if (nan || !(fabsf(ymax) < INFINITY)) return false;
+  const float D = fminf(ymax - ymin, kDTail);
+  rw = BucketRow<VEC>{a.logits + (long long)row * a.stride_bytes, a.vocab, T < 0.0f, aT, ymax,
+                      D > 0.0f ? fminf((float)kBk / D, 0x1p100f) : 0.0f};
+  return true;
+}
+
+// Chunk blockIdx.x of row blockIdx.y: its counts and masses, added to the
+// row's.
+template <bool VEC>
+__global__ void __launch_bounds__(kST) bucket_mass_kernel(ExactArgs a, BucketWs* ws) {
+  __shared__ BucketLds u;
+  BucketSmem& bs = u.bs;
+  const int row = a.row0 + blockIdx.y, tid = threadIdx.x;
+  BucketWs& w = ws[blockIdx.y];
+  BucketRow<VEC> rw;
+  if (!split_row<VEC>(a, w, row, rw)) return;  // uniform
+  for (int i = tid; i <= kBk; i += kST) bs.cur[i] = 0u;
+  for (int i = tid; i < kBk; i += kST) bs.inc[i] = 0ull;
+  __syncthreads();
+  int lo, hi;
+  split_chunk(a.vocab, lo, hi);
+  bucket_mass<VEC>(bs, rw, lo, hi);
+  __syncthreads();
+  for (int i = tid; i <= kBk; i += kST)
+    if (bs.cur[i]) atomicAdd(&w.cnt[i], bs.cur[i]);
+  for (int i = tid; i < kBk; i += kST)
+    if (bs.inc[i]) atomicAdd(&w.mass[i], bs.inc[i]);
+}
+
+// Chunk blockIdx.x of row blockIdx.y: its stored keys and its increments.
+template <bool VEC>
+__global__ void __launch_bounds__(kST) bucket_store_kernel(ExactArgs a, BucketWs* ws) {
+  __shared__ BucketLds u;
+  BucketSmem& bs = u.bs;
+  const int row = a.row0 + blockIdx.y, tid = threadIdx.x;
+  BucketWs& w = ws[blockIdx.y];
+  BucketRow<VEC> rw;
+  if (!split_row<VEC>(a, w, row, rw) || w.left) return;  // uniform
+  if (tid < 32) bs.exptab[tid] = kExp2Tab[tid];
+  {
+    unsigned st[kPerT];
+    short ev[kPerT];
+    unsigned char fv[kPerT];
+    take(w.start, st);
+    take(w.eg, ev);
+    take(w.flag, fv);
+    if (tid < 2) bs.start[kBk + tid] = w.start[kBk + tid];
+    put(bs.start, st);
+    put(bs.eg, ev);
+    put(bs.flag, fv);
+    for (int i = tid; i < kBk; i += kST) bs.inc[i] = 0ull;
+  }
+  __syncthreads();
+  int nbk, part, bA;
+  const int V = a.vocab;
+  bucket_cut(bs, a.top_k > 0 && a.top_k < V ? a.top_k : V, nbk, part);
+  bA = bucket_top(bs, nbk);
+  int lo, hi;
+  split_chunk(V, lo, hi);
+  uint32_t* K = a.scratch + (size_t)blockIdx.y * 2 * (size_t)V;
+  bucket_store<VEC, true>(bs, rw, lo, hi, nbk, bA, w.cur, w.topk, w.topi, K, K + V);
+  __syncthreads();
+  constexpr unsigned long long kWalk = 1ull << 63;
+  for (int i = tid; i < kBk; i += kST) {
+    const unsigned long long v = bs.inc[i];
+    if (v & ~kWalk) atomicAdd(&w.inc[i], v & ~kWalk);
+    if (v & kWalk) atomicOr(&w.inc[i], kWalk);
+  }
+}
+
 // The exp the exact path uses, for verification: out[i] = expf_glibc(in[i]).
 __global__ void expf_glibc_kernel(const float* in, float* out, long long n) {
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -3054,19 +3496,38 @@ __global__ void expf_glibc_kernel(const float* in, float* out, long long n) {
 constexpr size_t kExactScratch = 512ull << 20;
 
 template <int DT, bool VEC>
-void launch_exact_rows(const ExactArgs& a, int rows, hipStream_t stream) {
+void launch_exact_rows(const ExactArgs& a, int rows, hipStream_t stream, BucketWs* ws = nullptr,
+                       int G = 1) {
   if constexpr (DT == PKV_F32) {
     // sampled rows go to the buckets first; the rows they leave (a.fallback)
     // to the runs of equal values when every logit is a bf16 value, then to
     // the sort
     if (a.fallback) {
-      sample_bucket_kernel<VEC><<<rows, kST, 0, stream>>>(a);
-      sample_runs_kernel<DT, VEC><<<rows, kST, 0, stream>>>(a);
+      if (ws) {
+        const dim3 grid(G, rows);
+        bucket_extremes_kernel<VEC><<<grid, kST, 0, stream>>>(a, ws);
+        bucket_mass_kernel<VEC><<<grid, kST, 0, stream>>>(a, ws);
+        bucket_step_kernel<VEC, kRowPlan><<<rows, kST, 0, stream>>>(a, ws, G);
+        bucket_store_kernel<VEC><<<grid, kST, 0, stream>>>(a, ws);
+        bucket_step_kernel<VEC, kRowFinish><<<rows, kST, 0, stream>>>(a, ws, G);
+      } else {
+        sample_bucket_kernel<VEC><<<rows, kST, 0, stream>>>(a);
+      }
+      sample_left_kernel<VEC><<<rows, kST, 0, stream>>>(a);
+    } else {
+      sample_exact_kernel<DT, VEC><<<rows, kST, 0, stream>>>(a);
     }
-    sample_exact_kernel<DT, VEC><<<rows, kST, 0, stream>>>(a);
   } else {
     sample_runs_kernel<DT, VEC><<<rows, kST, 0, stream>>>(a);
   }
+}
+
+// Chunks per row of the f32 bucket path (1: one workgroup per row).
+int exact_split_groups(int batch, int vocab) {
+  if (vocab < kSplitMinVocab || batch > kSplitMaxRows) return 1;
+  const int g = std::min(std::min(256 / std::max(batch, 1), kMaxG),
+                         (vocab + kSplitMinChunk - 1) / kSplitMinChunk);
+  return std::max(g, 1);
 }
 
 template <int DT, bool VEC>
@@ -3084,9 +3545,13 @@ hipError_t launch_exact_dt(const ExactArgs& a0, int batch, hipStream_t stream) {
       DT == PKV_F32 ? std::max((size_t)2 * (size_t)a0.vocab * sizeof(uint32_t), runs_row)
                     : runs_row;
   const int rows = (int)std::max<size_t>(1, std::min<size_t>(batch, kExactScratch / per_row));
-  const size_t flags = DT == PKV_F32 ? (size_t)batch * sizeof(int32_t) : 0;
+  const size_t flags = DT == PKV_F32 ? ((size_t)batch * sizeof(int32_t) + 255) / 256 * 256 : 0;
+  // f32 batches that leave CUs idle with one workgroup per row: G chunks per
+  // row (every row in one launch then: rows == batch)
+  const int G = DT == PKV_F32 && rows == batch ? exact_split_groups(batch, a0.vocab) : 1;
+  const size_t split = G > 1 ? (size_t)batch * sizeof(BucketWs) : 0;
   void* p = nullptr;
-  hipError_t e = hipMallocAsync(&p, per_row * rows + flags, stream);
+  hipError_t e = hipMallocAsync(&p, per_row * rows + flags + split, stream);
   if (e != hipSuccess) return e;
   ExactArgs a = a0;
   a.scratch = static_cast<uint32_t*>(p);
@@ -3094,7 +3559,10 @@ hipError_t launch_exact_dt(const ExactArgs& a0, int batch, hipStream_t stream) {
     a.fallback = reinterpret_cast<int32_t*>(static_cast<char*>(p) + per_row * rows);
   for (int r0 = 0; r0 < batch; r0 += rows) {
     a.row0 = r0;
-    launch_exact_rows<DT, VEC>(a, std::min(rows, batch - r0), stream);
+    launch_exact_rows<DT, VEC>(
+        a, std::min(rows, batch - r0), stream,
+        G > 1 ? reinterpret_cast<BucketWs*>(static_cast<char*>(p) + per_row * rows + flags) : nullptr,
+        G);
   }
   e = hipGetLastError();
   const hipError_t f = hipFreeAsync(p, stream);

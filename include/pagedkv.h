@@ -506,7 +506,9 @@ int pkv_sample(const void* logits, int dtype, long long row_stride, int batch,
  * Scratch: 1 MB per row for f16/bf16 logits, 8 bytes per logit per row for
  * f32, at most 512 MB per launch (larger batches run in several launches),
  * in a stream-ordered allocation on `stream`.  One 1024-thread workgroup per
- * row. */
+ * row; at most 64 rows of at least 65,536 f32 logits take min(32, 256 /
+ * batch, ceil(vocab / 4096)) workgroups per row for the passes over the
+ * logits (five launches, 0.2 MB more scratch per row, the same tokens). */
 int pkv_sample_exact(const void* logits, int dtype, long long row_stride, int batch,
                      int vocab, const float* temperatures, int top_k, float top_p,
                      uint64_t seed, int32_t* tokens, void* stream);

@@ -515,3 +515,32 @@ def test_exact_f32_buckets_agree_with_the_sort_on_shuffled_rows(gpu):
     picked = {float(base[perms[b][got[b]]]) for b in range(B)}
     assert len(picked) == 1, picked
     assert got == [oracle.sample(x[b], 0.8, top_p=0.9)[0] for b in range(B)]
+
+
+@pytest.mark.parametrize("V", [65536, 65539, 131073])
+@pytest.mark.parametrize("top_k,top_p", [(None, None), (700, None), (None, 0.95)])
+def test_exact_f32_split_rows_equal_whole_rows(gpu, V, top_k, top_p):
+    # batches of at most 64 rows of at least 65,536 f32 logits take several
+    # workgroups per row; the same rows in a batch of 65 take one each.  Every
+    # kind of row: sampled at either sign of the temperature, greedy, with a
+    # NaN, an infinity, -inf entries, equal values, and one dominant token
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((13, V)) * 3).astype(np.float32)
+    x[3, 17], x[4, V - 1], x[5, ::3] = np.nan, np.inf, -np.inf
+    x[6] = np.round(x[6])
+    x[7] = 0.25
+    x[8, V // 2] = 40.0
+    x[9, :] = -np.inf
+    x[10] *= 1e-3
+    temps = np.array([0.7, -1.3, 0.0, 0.0, 0.0, 1.0, 0.9, 1.0, 0.5, 0.0, 2.0, 0.3, 1.0], np.float32)
+    lg, t = torch.from_numpy(x).to(gpu), torch.from_numpy(temps).to(gpu)
+    whole = pagedkv.sample(lg.repeat(5, 1), t.repeat(5), top_k=top_k, top_p=top_p)
+    for n in (1, 2, 13):
+        for r0 in range(0, 13 - n + 1, n):
+            got = pagedkv.sample(lg[r0:r0 + n].contiguous(), t[r0:r0 + n].contiguous(),
+                                 top_k=top_k, top_p=top_p)
+            assert got.tolist() == whole[r0:r0 + n].tolist(), (n, r0)
+    got = pagedkv.sample(lg.repeat(5, 1)[:64], t.repeat(5)[:64], top_k=top_k, top_p=top_p)
+    assert got.tolist() == whole[:64].tolist()
+    want = [oracle.sample(x[b], float(temps[b]), top_k=top_k, top_p=top_p)[0] for b in (0, 1, 5, 6, 8)]
+    assert whole[[0, 1, 5, 6, 8]].tolist() == want
