@@ -56,11 +56,14 @@ struct DCfg {
   // against 406-411 us, Llama-3-70B 449 against 460 us, Llama-3.2-1B 8.5
   // against 8.7-8.8 us).  The RoPE kernels (more registers live around the
   // loop) measured the other way (410 against 400 us) and keep 64 tokens
-  // below GQA 8, and 48 for bf16 rows of 128 at GQA 8.
+  // below GQA 8.  At GQA 8 with bf16 rows of 128, tiles of 48 / 32 / 16 tokens
+  // (two waves per SIMD; fewer registers with 16) ran 3 sequences of 16-30k
+  // tokens in 79.5 / 74.3 / 72.9 us, 4 of 8-16k in 54.9 / 51.7 / 47.8, 32 of
+  // 1-4k in 84.8 / 82.7 / 82.6 and 128 of 0.5-4k in 218 / 215.4 / 216: 16.
   static constexpr int NSTMAX =
       (R >= 16  ? 16
        : !ROPE  ? 32
-       : R >= 8 ? (DT == PKV_BF16 && HD == 128 ? 48 : 32)
+       : R >= 8 ? (DT == PKV_BF16 && HD == 128 ? 16 : 32)
                 : PKV_DECODE_TILE) /
       16;
   static constexpr int NST = NST0 < 1 ? 1 : (NST0 > NSTMAX ? NSTMAX : NST0);  // sub-tiles
