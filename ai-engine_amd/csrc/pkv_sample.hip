@@ -1604,8 +1604,12 @@ struct RunSmem {
 // (the running-sum walks read them one at a time, in order).
 constexpr int kLdsRuns = 4096;
 
+// The one-pass histogram's words are padded by one in 32: a thread reads 32
+// consecutive words, which would put a wave's 64 lanes on two banks (a
+// 32-way conflict: 15 of the 100 us of 256 rows).
+__device__ __forceinline__ uint32_t hist_at(uint32_t w) { return w + (w >> 5); }
 union RunLds {
-  unsigned int hist[kHalfKeys];
+  unsigned int hist[kHalfKeys + kHalfKeys / 32];
   struct {
     SampleSmem sm;
     RunSmem rs;
@@ -1897,8 +1901,9 @@ __device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
   // 65,535 logits).
   int R = 0;
   bool two_pass = false;
+  bool in_lds = false;  // the runs lie in LDS
   {
-    for (int b = tid; b < kHalfKeys; b += kST) u.hist[b] = 0u;
+    for (int b = tid; b < kHalfKeys + kHalfKeys / 32; b += kST) u.hist[b] = 0u;
     __syncthreads();
     bool inexact = false;
     for_each<DT, VEC, kRowBatch>(x, V, [&](int, float v) {
@@ -1908,9 +1913,9 @@ __device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
       const uint32_t k0 = __builtin_amdgcn_readfirstlane(k);
       const uint32_t sh = (k & 1u) * 16u;
       if (__ballot(k == k0) == act) {  // one key across the wave: one addition
-        if (lane == __builtin_ctzll(act)) atomicAdd(&u.hist[k >> 1], (unsigned)__popcll(act) << sh);
+        if (lane == __builtin_ctzll(act)) atomicAdd(&u.hist[hist_at(k >> 1)], (unsigned)__popcll(act) << sh);
       } else {
-        atomicAdd(&u.hist[k >> 1], 1u << sh);
+        atomicAdd(&u.hist[hist_at(k >> 1)], 1u << sh);
       }
     });
     if constexpr (DT == PKV_F32) {
@@ -1921,18 +1926,26 @@ __device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
       __syncthreads();
     }
     const int whi = kHalfKeys - 1 - 32 * tid;  // this thread's 32 words (64 keys), descending
+    unsigned int hw[32];
     unsigned int nz = 0, sum = 0;
+#pragma unroll
     for (int j = 0; j < 32; ++j) {
-      const unsigned int w = u.hist[whi - j];
+      const unsigned int w = u.hist[hist_at((uint32_t)(whi - j))];
+      hw[j] = w;
       nz += (w >> 16 != 0u) + ((w & 0xffffu) != 0u);
       sum += (w >> 16) + (w & 0xffffu);
     }
     unsigned int total, counted;
     unsigned int at = block_excl_scan(nz, wtmp, total);
     block_excl_scan(sum, wtmp, counted);
-    if (counted == (unsigned int)V) {
+    if (counted == (unsigned int)V) {  // uniform; every thread has read its words
+      if (total <= (unsigned int)kLdsRuns) {
+        ra = RunArrays{u.x.key, u.x.cnt, u.x.start, u.x.val};
+        in_lds = true;
+      }
+#pragma unroll
       for (int j = 0; j < 32; ++j) {
-        const unsigned int w = u.hist[whi - j];
+        const unsigned int w = hw[j];
         const uint32_t kh = 2u * (uint32_t)(whi - j) + 1u;
         if (w >> 16) {
           ra.key[at] = kh;
@@ -1948,7 +1961,7 @@ __device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
       R = (int)total;
     }
     two_pass = counted != (unsigned int)V;
-    __syncthreads();  // every thread has read the histogram before it is cleared or reused
+    __syncthreads();  // the runs are written; the histogram may be cleared
   }
   for (int half = 1; half >= 0 && two_pass; --half) {
     for (int b = tid; b < kHalfKeys; b += kST) u.hist[b] = 0u;
@@ -2004,7 +2017,7 @@ __device__ __forceinline__ void runs_row(const ExactArgs& a, RunLds& u) {
     __syncthreads();
     R = rs.R;
   }
-  if (R <= kLdsRuns) {  // the runs move to LDS: the walks below read them one by one
+  if (!in_lds && R <= kLdsRuns) {  // the runs move to LDS: the walks below read them one by one
     for (int r = tid; r < R; r += kST) {
       u.x.key[r] = ra.key[r];
       u.x.cnt[r] = ra.cnt[r];
