@@ -177,6 +177,12 @@ int pkv_pool_create(pkv_pool** out, int n_layers, int num_blocks,
   }
   void* base = nullptr;
   hipError_t e = hipMalloc(&base, total);
+  if (e == hipErrorOutOfMemory) {  // without the scratch that sampling keeps
+    (void)hipGetLastError();
+    (void)hipDeviceSynchronize();
+    pkv::scratch_trim(device);
+    e = hipMalloc(&base, total);
+  }
   if (e != hipSuccess) {
     delete p;
     return fail(nullptr, PKV_ERR_OOM, "pool hipMalloc(%zu bytes): %s", total, hipGetErrorString(e));
@@ -1022,6 +1028,16 @@ int pkv_rope_check(pkv_rope* r) {
   if (e == hipSuccess && bits) e = hipMemset(r->err, 0, 4);
   if (e != hipSuccess) return hip_fail(nullptr, e, "rope check");
   if (bits) return fail(nullptr, PKV_ERR_DEVICE_DATA, "rope: position outside the table");
+  return PKV_OK;
+}
+
+int pkv_sample_trim(void) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e != hipSuccess)
+    return fail(nullptr, PKV_ERR_HIP, "sample_trim: %s", hipGetErrorString(e));
+  pkv::scratch_trim(dev);
   return PKV_OK;
 }
 

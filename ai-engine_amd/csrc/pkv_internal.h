@@ -88,6 +88,8 @@ inline size_t dtype_bytes(int dt) { return dt == PKV_F32 ? 4 : 2; }
 // Token selection (pkv_sample.hip): the fixed draw r of a seed, and the
 // launcher of the per-row argmax / sample kernel.
 float sample_draw(uint64_t seed);
+// Returns the free memory of the sampling calls' pool on `device`.
+void scratch_trim(int device);
 hipError_t launch_sample(const void* logits, int dtype, long long row_stride, int batch,
                          int vocab, const float* temperatures, int top_k, float top_p,
                          float r, int32_t* tokens, hipStream_t stream);

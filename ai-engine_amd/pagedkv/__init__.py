@@ -162,9 +162,9 @@ def sample(logits, temperatures=None, top_k: int | None = None, top_p: float | N
     temperatures: (batch,) float32 on the device (None: all greedy).
     exact=True (pkv_sample_exact, the default since the engine needs the
     reference's tokens): the reference's f32 arithmetic bit for bit, so the
-    token is the reference's on every row.  It allocates its scratch on the
-    stream for each call (hipMallocAsync, freed in stream order after the
-    launch): 1 MiB per row for 16-bit logits (the row's runs of equal
+    token is the reference's on every row.  It takes its scratch on the
+    stream for each call (freed in stream order after the launch; the library
+    keeps up to 512 MiB of it per device until sample_trim()): 1 MiB per row for 16-bit logits (the row's runs of equal
     values); for f32 logits 8 bytes per logit (1 MiB per 128k-entry row),
     rows taken in rounds of at most 512 MiB.  top_p=None is the reference's
     None (no cut; passed as NaN), which differs from Some(1.0): with f32
@@ -214,6 +214,12 @@ def sample(logits, temperatures=None, top_k: int | None = None, top_p: float | N
                  _dev_ptr(t) if t is not None else None, top_k or 0, tp, seed, _dev_ptr(out),
                  *extra, _stream_ptr(s)), None)
     return out
+
+
+def sample_trim() -> None:
+    """Gives back the scratch that sample() keeps on the current device (at
+    most 512 MiB; pkv_sample_trim)."""
+    check(lib().pkv_sample_trim(), None)
 
 
 def sample_expf(x):

@@ -113,6 +113,7 @@ SIGNATURES: dict[str, tuple] = {
     "pkv_sample_exact_routes": (_I, [_P, _I, ctypes.c_longlong, _I, _I, _P, _I, ctypes.c_float,
                                      ctypes.c_uint64, _P, _P, _P]),
     "pkv_sample_expf": (_I, [_P, _P, ctypes.c_longlong, _P]),
+    "pkv_sample_trim": (_I, []),
     "pkv_sample_draw": (ctypes.c_float, [ctypes.c_uint64]),
     "pkv_pool_profile": (_I, [_P, _I]),
     "pkv_pool_profile_read": (_I, [_P, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_I)]),

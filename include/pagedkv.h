@@ -484,8 +484,10 @@ int pkv_append_rope(pkv_pool* pool, int layer, const pkv_rope* rope,
  * each row over G = min(32, 256 / batch, ceil(vocab / 4096)) workgroups,
  * with 57,624 + 4,096 G bytes per row of partial histograms (at most 184 KiB
  * per row; 1.5 MB for 8 rows, 8.4 MB for 128) in a stream-ordered allocation
- * on `stream` (hipMallocAsync / hipFreeAsync, capturable in a HIP graph); if
- * that allocation fails, one workgroup per row.  Both give the same tokens. */
+ * on `stream` (capturable in a HIP graph); if that allocation fails, one
+ * workgroup per row.  Both give the same tokens.  Scratch of this call and of
+ * pkv_sample_exact comes from a memory pool of the library, which keeps up to
+ * 512 MiB per device for the next call until pkv_sample_trim. */
 int pkv_sample(const void* logits, int dtype, long long row_stride, int batch,
                int vocab, const float* temperatures, int top_k, float top_p,
                uint64_t seed, int32_t* tokens, void* stream);
@@ -505,7 +507,8 @@ int pkv_sample(const void* logits, int dtype, long long row_stride, int batch,
  * sum, the r threshold) takes exactly the reference's rounding steps.
  * Scratch: 1 MB per row for f16/bf16 logits, 8 bytes per logit per row for
  * f32, at most 512 MB per launch (larger batches run in several launches),
- * in a stream-ordered allocation on `stream`.  One 1024-thread workgroup per
+ * in a stream-ordered allocation on `stream` (kept as pkv_sample's is, at most
+ * 512 MiB in all until pkv_sample_trim).  One 1024-thread workgroup per
  * row; at most 64 rows of at least 65,536 f32 logits take min(32, 256 /
  * batch, ceil(vocab / 4096)) workgroups per row for the passes over the
  * logits (five launches, 0.2 MB more scratch per row, the same tokens). */
@@ -526,6 +529,10 @@ int pkv_sample_exact_routes(const void* logits, int dtype, long long row_stride,
  * counterpart): out[i] = expf(in[i]) as glibc computes it; device arrays of
  * n floats, on `stream`. */
 int pkv_sample_expf(const float* in, float* out, long long n, void* stream);
+/* Gives back the free scratch that pkv_sample and pkv_sample_exact keep on the
+ * calling thread's current device (waits for the device; the next call
+ * allocates again).  pkv_pool_create does the same when memory runs out. */
+int pkv_sample_trim(void);
 /* StdRng::seed_from_u64(seed).gen::<f32>() (sample.rs:41-42; host only). */
 float pkv_sample_draw(uint64_t seed);
 

@@ -544,3 +544,44 @@ def test_exact_f32_split_rows_equal_whole_rows(gpu, V, top_k, top_p):
     assert got.tolist() == whole[:64].tolist()
     want = [oracle.sample(x[b], float(temps[b]), top_k=top_k, top_p=top_p)[0] for b in (0, 1, 5, 6, 8)]
     assert whole[[0, 1, 5, 6, 8]].tolist() == want
+
+
+def test_kept_scratch_serves_streams_and_threads_and_is_given_back(gpu):
+    # the scratch pool outlives a call: calls of different sizes from two
+    # threads on streams of their own, some with a synchronisation after each,
+    # give the tokens of calls made alone; what is kept stays below 512 MiB
+    # and goes back to the device with sample_trim
+    import threading
+    rng = np.random.default_rng(21)
+    x = torch.from_numpy(_rows(rng, 96, 70001).astype(np.float32)).to(gpu)
+    cases = [(x[:96].to(torch.bfloat16), True), (x[:5], True), (x[:70], True),
+             (x[:9].to(torch.float16), False)]
+    temps = torch.full((96,), 0.9, device=gpu)
+
+    def sample(lg, exact):
+        return pagedkv.sample(lg, temps[:len(lg)], exact=exact)
+
+    want = [sample(*c).tolist() for c in cases]
+    bad = []
+
+    def work(sync):
+        with torch.cuda.stream(torch.cuda.Stream()) as _:
+            torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+            for i in range(3):
+                got = [sample(*c) for c in cases]
+                if sync:
+                    torch.cuda.synchronize()
+                bad.extend((i, j) for j, w in enumerate(want) if got[j].tolist() != w)
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in (False, True)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
+    torch.cuda.synchronize()
+    kept = torch.cuda.mem_get_info()[0]
+    pagedkv.sample_trim()
+    freed = torch.cuda.mem_get_info()[0] - kept
+    assert (60 << 20) <= freed <= (520 << 20), freed   # at least 70 rows of 1 MiB less rounding
+    assert [sample(*c).tolist() for c in cases] == want
