@@ -585,3 +585,19 @@ def test_kept_scratch_serves_streams_and_threads_and_is_given_back(gpu):
     freed = torch.cuda.mem_get_info()[0] - kept
     assert (60 << 20) <= freed <= (520 << 20), freed   # at least 70 rows of 1 MiB less rounding
     assert [sample(*c).tolist() for c in cases] == want
+
+
+@pytest.mark.parametrize("V", [1000, 40000, 131072])
+@pytest.mark.parametrize("values", [1, 2, 7, 60])
+def test_exact_runs_of_many_copies(gpu, V, values):
+    # few distinct 16-bit logits, so runs of up to V copies that cross several
+    # binades and reach the threshold (r, top_p) inside a run
+    rng = np.random.default_rng(V + values)
+    x = torch.from_numpy(rng.choice(rng.uniform(-6, 6, values), (4, V)).astype(np.float32))
+    x = x.to(torch.bfloat16)
+    temps = np.array([0.6, 1.0, -0.8, 2.5], np.float32)
+    for top_p in (None, 0.5):
+        got = pagedkv.sample(x.to(gpu), torch.from_numpy(temps).to(gpu), top_p=top_p).tolist()
+        want = [oracle.sample(x[b].float().numpy(), float(temps[b]), top_p=top_p)[0]
+                for b in range(4)]
+        assert got == want, top_p
