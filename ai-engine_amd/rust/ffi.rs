@@ -269,6 +269,7 @@ extern "C" {
     pub fn pkv_sample_expf(
         in: *const f32, out: *mut f32, n: c_longlong, stream: *mut c_void
     ) -> c_int;
+    pub fn pkv_sample_trim() -> c_int;
     pub fn pkv_sample_draw(seed: u64) -> f32;
 
     // ---- block allocator and tables (block_table.rs:5-58)
