@@ -109,7 +109,8 @@ __device__ __forceinline__ void exotic_rows(const PrefillKArgs& a, int R, int g,
       s *= a.scale_log2;
       const float mn = s > m ? s : m;  // a NaN score leaves m and makes the weights NaN
       const float al = m == mn ? 1.0f : fast_exp2(m - mn);
-      const float w = fast_exp2(s - mn);
+      // weight 0 also before the first finite score (m = mn = -inf)
+      const float w = s == -INFINITY ? 0.0f : fast_exp2(s - mn);
       m = mn;
       l = l * al + w;
       for (int d = 0; d < ND; ++d) o[d] = fmaf(w, vr[lane + 64 * d], o[d] * al);
@@ -394,13 +395,14 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   }
   {
     // a sum that is not finite: a value whose split overflowed (or an infinity
-    // or NaN in the inputs)
+    // or NaN in the inputs); or no weight in group 0, which every row sees: its
+    // products all overflowed to -inf (the merge below needs a finite m there)
     float z = l;
 #pragma unroll
     for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) z = fmaf(o[dt][r], 0.0f, z);
-    if (has_rows && !(fabsf(z) < INFINITY)) not_finite = 1;
+    if (has_rows && (!(fabsf(z) < INFINITY) || (kg == 0 && l == 0.0f))) not_finite = 1;
   }
   constexpr int kXW = (C::NDT * 16 + 2) * 64;  // floats per row group
   static_assert(RG * kXW * 4 <= 2 * C::STAGE, "");

@@ -337,3 +337,53 @@ def test_f32_split_values_beyond_bf16(gpu):
     scale = np.maximum(np.abs(ref[fin]), np.abs(vp[np.abs(vp) < 1e38]).max())
     assert (np.abs(got[fin] - ref[fin]) <= 4e-6 * scale).all()
     c.close()
+
+
+@pytest.mark.parametrize("product", [False, True])
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("prior,chunk,keys", [
+    (0, 90, [0]),                       # the first key of all
+    (0, 90, range(32)),                 # the first key group's step
+    (0, 90, range(70)),                 # rows with no finite score (NaN), rows with some
+    (1100, 40, [1024]),                 # the first key of the second part
+    (1100, 40, range(1024)),            # a whole part
+    (2200, 40, [0, *range(1024, 2048)]),
+    (1100, 40, [0, 1024, 1100, 1105]),  # and keys of the chunk itself
+])
+def test_f32_split_minus_infinity_scores(gpu, prior, chunk, keys, fused, product):
+    # keys of score -inf (an infinity in K, or a product of finite values that
+    # overflows) have weight 0 wherever they stand; a row all of whose scores
+    # are -inf is NaN, as in the reference
+    c = PCase(gpu, wl.F32, 4, 2, 64, 16, [prior, 3], [chunk, 20], seed=prior + len(keys))
+    big = 2.0 ** 70 if product else 1.0
+    c.q[:, :, 0] = big * (1.0 + (c.q[:, :, 0] > 0))
+    c.kp[..., 0] = 0.0
+    for key in keys:
+        c.kp[c.tables[0, key // 16], key % 16, :, 0] = -big if product else -np.inf
+    c.cache.write_bytes(0, pagedkv.K, c.kp)
+    if fused:  # the chunk's rows from the call, other values in the pool
+        sl = _slots(c)
+        flat = lambda a: a.reshape(-1, 2, 64)
+        kn, vn = flat(c.kp)[sl].copy(), flat(c.vp)[sl].copy()
+        kz, vz = c.kp.copy(), c.vp.copy()
+        flat(kz)[sl], flat(vz)[sl] = 3.0, 5.0
+        c.cache.write_bytes(0, pagedkv.K, kz)
+        c.cache.write_bytes(0, pagedkv.V, vz)
+        dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+        got = c.cache.layer(0).prefill_attention(
+            dev(c.q), dev(c.cu), dev(c.ctx), dev(c.tables), max_q_len=chunk,
+            max_context_len=int(c.ctx.max()), scale=c.scale, out_dtype=torch.float32,
+            k_new=dev(kn), v_new=dev(vn)).cpu().numpy()
+        c.cache.check()
+    else:
+        got = c.run()
+    if product:  # in 64 bits the product is finite: the reference's -inf
+        c.q[:, :, 0], c.kp[..., 0] = 1.0, np.where(c.kp[..., 0] < 0, -np.inf, 0.0)
+    ref = c.reference()
+    fin = np.isfinite(ref)
+    # (without a prior, token 0 sees key 0 alone)
+    assert np.isnan(got[~fin]).all() and fin.all() == (prior > 0)
+    # the bound of test_f32_split_products, with a row's sums of up to 2,240
+    # keys in one chain: 2,240 roundings of 2^-24 at random, below 2.9e-6
+    assert np.abs(got - ref)[fin].max() <= 7e-6 * np.abs(c.vp).max()
+    c.close()
