@@ -29,9 +29,9 @@
 // the score MFMAs, or 64 rows per workgroup gave the same or longer times.
 //
 // The split of a value beyond bf16's range (|x| > 3.39e38, infinities) leaves
-// NaN in its remainders, so every sum it enters ends as NaN: a workgroup whose
-// sums are not all finite recomputes its rows from the f32 values on the VALU
-// (exotic_rows), and such inputs give what f32 arithmetic gives.
+// NaN in its remainders, so every sum it enters ends as NaN: rows whose sums
+// are not all finite are computed again from the f32 values on the f32 MFMA,
+// and such inputs give what f32 arithmetic gives.
 #include <type_traits>
 
 #include "pkv_prefill_dev.h"
@@ -55,7 +55,12 @@ struct SCfg {
   static constexpr int STAGE = 2 * GRP;         // both key groups
   static constexpr int NDT = HD / 32;           // 32-dim tiles of O^T
   static constexpr int NKQ = HD / 16;           // 16-dim steps of Q K^T
+  // rows computed again in f32: K and V as they are, the weights of a wave
+  static constexpr int KP32 = RB + 16, VP32 = RB + 32;  // row pitches
+  static constexpr int STAGE32 = kSKeys * (KP32 + VP32);
+  static constexpr int P32 = 32 * 32 * 4;
   static_assert(kSKeys * CH % NT == 0, "");
+  static_assert(2 * STAGE32 + 2 * RG * P32 <= 2 * STAGE, "the f32 rows fit the bf16 planes' LDS");
 };
 
 // Four floats to three bf16 planes (round to nearest even; remainders are
@@ -82,59 +87,15 @@ __device__ __forceinline__ void mfma32b(const u32x4& a, const u32x4& b, f32x16& 
                                                 __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
 }
 
-// Rows of a workgroup whose sums were not finite, in plain f32: one row
-// per wave at a time, lane = dims lane, lane + 64, ..
-template <int HD, int RG, typename RowPtr>
-__device__ __forceinline__ void exotic_rows(const PrefillKArgs& a, int R, int g, int q0,
-                                                      int prior, int row0, int n_rows, int k_lo,
-                                                      int k_hi, bool partial, size_t item,
-                                                      RowPtr row_ptr) {
-  constexpr int ND = HD / 64;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int H = a.kvh * R;
-  for (int rr = wave; rr < 32 * RG; rr += 2 * RG) {
-    const int r = row0 + rr;
-    if (r >= n_rows) break;
-    const float* q = reinterpret_cast<const float*>(a.q) +
-                     ((size_t)(q0 + r / R) * H + g * R + r % R) * HD;
-    float m = -INFINITY, l = 0.0f, o[ND];
-    for (int d = 0; d < ND; ++d) o[d] = 0.0f;
-    const int kend = min(k_hi, prior + r / R + 1);
-    for (int k = k_lo; k < kend; ++k) {
-      const float *kr, *vr;
-      row_ptr(k, kr, vr);
-      float s = 0.0f;
-      for (int d = 0; d < ND; ++d) s = fmaf(q[lane + 64 * d], kr[lane + 64 * d], s);
-      for (int x = 1; x < 64; x <<= 1) s += shfl_xor_f(s, x);
-      s *= a.scale_log2;
-      const float mn = s > m ? s : m;  // a NaN score leaves m and makes the weights NaN
-      const float al = m == mn ? 1.0f : fast_exp2(m - mn);
-      // weight 0 also before the first finite score (m = mn = -inf)
-      const float w = s == -INFINITY ? 0.0f : fast_exp2(s - mn);
-      m = mn;
-      l = l * al + w;
-      for (int d = 0; d < ND; ++d) o[d] = fmaf(w, vr[lane + 64 * d], o[d] * al);
-    }
-    if (partial) {
-      const size_t pr = item * (32 * RG) + rr;
-      for (int d = 0; d < ND; ++d) a.part_o[pr * HD + lane + 64 * d] = o[d];
-      if (lane == 0) {
-        a.part_ml[2 * pr] = m;
-        a.part_ml[2 * pr + 1] = l;
-      }
-    } else {
-      float* out = reinterpret_cast<float*>(a.out) +
-                   ((size_t)(q0 + r / R) * H + g * R + r % R) * HD;
-      for (int d = 0; d < ND; ++d) out[lane + 64 * d] = o[d] / l;
-    }
-  }
+__device__ __forceinline__ void mfma32f(float a, float b, f32x16& acc) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
 }
 
 template <int HD, int RG, bool FUSED>
 __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a) {
   using C = SCfg<HD, RG>;
   __shared__ __attribute__((aligned(16))) char lds[2 * C::STAGE];
-  __shared__ int not_finite;
+  __shared__ uint32_t again[RG];  // rows to compute again in f32, a bit each
 
   const int R = a.rq;
   const int tid = threadIdx.x;
@@ -175,7 +136,7 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   if constexpr (FUSED)
     prefill_store_chunk<C::ROWS, C::RB, C::NT>(a, R, rb, n_rows, q_len, prior, q0,
                                                   part == nparts - 1, table, kh, vh, kin, vin);
-  if (tid == 0) not_finite = 0;
+  if (tid < RG) again[tid] = 0u;
 
   const int k_hi = part + 1 < nparts ? (part + 1) * a.part_keys : n_keys;
   const int t_lo = part * (a.part_keys / kSKeys);
@@ -188,7 +149,7 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   const int rc = min(roww + c32, n_rows - 1);
   const int lim = prior + rc / R;
 
-  // ---- loads: chunk i of a thread is key (tid / CH) + (kSThreads / CH) i of
+  // ---- loads: chunk i of a thread is key (tid / CH) + (NT / CH) i of
   //      the step, bytes 16 (tid % CH); keys past n_keys are clamped.  The
   //      block id of each is read one step before its rows. ----
   const int lkey = tid / C::CH;
@@ -387,80 +348,193 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   }
   if (bad_block) atomicOr(a.err, PKV_EBIT_BLOCK);
 
-  // ---- merge of the two key groups: group 1 hands (m, l, O) over in LDS,
-  //      each register 64 lanes wide (no bank conflicts) ----
-  {
+  // ---- rows to compute again: a sum that is not finite (a value whose split
+  //      overflowed, or an infinity or NaN in the inputs), or no weight in key
+  //      group 0, which every row sees (its products all overflowed to -inf) ----
+  auto full_sum = [&]() __attribute__((always_inline)) {  // both halves' part of l
     const auto lw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(lw[0]) + __uint_as_float(lw[1]);
-  }
+  };
+  full_sum();
   {
-    // a sum that is not finite: a value whose split overflowed (or an infinity
-    // or NaN in the inputs); or no weight in group 0, which every row sees: its
-    // products all overflowed to -inf (the merge below needs a finite m there)
     float z = l;
 #pragma unroll
     for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) z = fmaf(o[dt][r], 0.0f, z);
-    if (has_rows && (!(fabsf(z) < INFINITY) || (kg == 0 && l == 0.0f))) not_finite = 1;
+    const unsigned long long w = __builtin_amdgcn_ballot_w64(
+        roww + c32 < n_rows && (!(fabsf(z) < INFINITY) || (kg == 0 && l == 0.0f)));
+    if (w && lane == 0) atomicOr(&again[rw], (uint32_t)w | (uint32_t)(w >> 32));
   }
+
+  // ---- merge of the two key groups: group 1 hands (m, l, O) over in LDS,
+  //      each register 64 lanes wide (no bank conflicts) ----
   constexpr int kXW = (C::NDT * 16 + 2) * 64;  // floats per row group
   static_assert(RG * kXW * 4 <= 2 * C::STAGE, "");
   float* xo = reinterpret_cast<float*>(lds) + rw * kXW;
-  if (kg == 1) {
+  const bool partial = nparts > 1;
+  const size_t item = ((size_t)sg * a.row_blocks + rb) * a.max_parts + part;
+  auto hand_over = [&]() __attribute__((always_inline)) {
+    if (kg == 1) {
+#pragma unroll
+      for (int dt = 0; dt < C::NDT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *reinterpret_cast<f32x4*>(xo + ((dt * 4 + r / 4) * 64 + lane) * 4) =
+              f32x4{o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]};
+      xo[C::NDT * 16 * 64 + lane] = m;
+      xo[C::NDT * 16 * 64 + 64 + lane] = l;
+    }
+    __syncthreads();
+  };
+  auto merge_store = [&](uint32_t rows) __attribute__((always_inline)) {  // bit c32: row roww + c32
+    if (kg == 1) return;
+    const float m1 = xo[C::NDT * 16 * 64 + lane], l1 = xo[C::NDT * 16 * 64 + 64 + lane];
+    const float M = fmaxf(m, m1);
+    // (m = m1 = -inf: no finite score, sums of 0)
+    const float w0 = m == M ? 1.0f : fast_exp2(m - M), w1 = m1 == M ? 1.0f : fast_exp2(m1 - M);
+    l = l * w0 + l1 * w1;
+    const int r = roww + c32;
+    if (r >= n_rows || !((rows >> c32) & 1u)) return;
+    const float f0 = partial ? w0 : w0 / l, f1 = partial ? w1 : w1 / l;
+    const size_t pr = item * C::ROWS + (r - row0);
+    float* dst = partial ? a.part_o + pr * HD
+                         : reinterpret_cast<float*>(a.out) +
+                               ((size_t)(q0 + r / R) * H + g * R + r % R) * HD;
 #pragma unroll
     for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; r += 4)
-        *reinterpret_cast<f32x4*>(xo + ((dt * 4 + r / 4) * 64 + lane) * 4) =
-            f32x4{o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]};
-    xo[C::NDT * 16 * 64 + lane] = m;
-    xo[C::NDT * 16 * 64 + 64 + lane] = l;
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(xo + ((dt * 4 + q4) * 64 + lane) * 4);
+        f32x4 y;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = o[dt][4 * q4 + j] * f0 + x[j] * f1;
+        *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * q4 + 4 * hh) = y;
+      }
+    if (partial && hh == 0) {
+      a.part_ml[2 * pr] = M;
+      a.part_ml[2 * pr + 1] = l;
+    }
+  };
+  hand_over();
+  const uint32_t mine = (uint32_t)__builtin_amdgcn_readfirstlane((int)again[rw]);
+  uint32_t any = 0;
+#pragma unroll
+  for (int i = 0; i < RG; ++i) any |= again[i];
+  merge_store(~mine);
+  if (__builtin_amdgcn_readfirstlane((int)any) == 0) return;  // workgroup-uniform
+
+  // ---- rows `mine` again on the f32 MFMA, with the same split of rows and
+  //      keys over the waves: K and V in LDS as they are (double-buffered),
+  //      the running maximum exact (a weight above 1 could overflow a large
+  //      value).  One prompt of 4,096 tokens (14 query heads on 2) whose first
+  //      key holds a NaN: 531 us (205 without it), against 26,200 with a row
+  //      per wave and a key at a time on the VALU. ----
+  float qs[HD / 2];  // Q[row c32][HD / 2 hh ..], the B operand
+  {
+    const char* qrow = a.q + ((size_t)(q0 + rc / R) * H + g * R + rc % R) * C::RB + C::RB / 2 * hh;
+#pragma unroll
+    for (int i = 0; i < HD / 8; ++i) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(qrow + 16 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qs[4 * i + j] = x[j];
+    }
   }
-  __syncthreads();
-  const size_t item = ((size_t)sg * a.row_blocks + rb) * a.max_parts + part;
-  if (not_finite) {  // workgroup-uniform
-    exotic_rows<HD, RG>(a, R, g, q0, prior, row0, n_rows, t_lo * kSKeys, k_hi, nparts > 1, item,
-                           [&](int key, const float*& kr, const float*& vr) {
-                             const bool fresh = FUSED && key >= prior;
-                             const int blk = fresh ? 0 : table[key >> a.bs_log2];
-                             const bool bad = (unsigned)blk >= (unsigned)a.num_blocks;
-                             const size_t off =
-                                 fresh ? (size_t)(q0 + key - prior) * slot_stride
-                                       : (size_t)(bad ? 0 : blk) * blk_stride +
-                                             (size_t)(key & tmask) * slot_stride;
-                             kr = reinterpret_cast<const float*>((fresh ? kin : kh) + off);
-                             vr = reinterpret_cast<const float*>((fresh ? vin : vh) + off);
-                           });
-    return;
-  }
-  if (kg == 1 || !has_rows) return;
-  const float m1 = xo[C::NDT * 16 * 64 + lane], l1 = xo[C::NDT * 16 * 64 + 64 + lane];
-  const float M = fmaxf(m, m1);  // finite: key group 0 holds the part's first key
-  const float w0 = fast_exp2(m - M), w1 = fast_exp2(m1 - M);
-  l = l * w0 + l1 * w1;
-  const int r = roww + c32;
-  if (r >= n_rows) return;
-  const bool partial = nparts > 1;
-  const float f0 = partial ? w0 : w0 / l, f1 = partial ? w1 : w1 / l;
-  const size_t pr = item * C::ROWS + (r - row0);
-  float* dst = partial ? a.part_o + pr * HD
-                       : reinterpret_cast<float*>(a.out) +
-                             ((size_t)(q0 + r / R) * H + g * R + r % R) * HD;
+  m = -INFINITY;
+  l = 0.0f;
 #pragma unroll
   for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(xo + ((dt * 4 + q4) * 64 + lane) * 4);
-      f32x4 y;
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+  auto again_step = [&](int t) __attribute__((always_inline)) {
+    const char* base = lds + (t & 1) * C::STAGE32;
+    const char* kl = base + (32 * kg + c32) * C::KP32 + C::RB / 2 * hh;
+    const char* vl = base + kSKeys * C::KP32 + 32 * kg * C::VP32;
+    const int k0 = t * kSKeys + 32 * kg;
+    f32x16 sc;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = o[dt][4 * q4 + j] * f0 + x[j] * f1;
-      *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * q4 + 4 * hh) = y;
+    for (int r = 0; r < 16; ++r) sc[r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < HD / 8; ++i) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(kl + 16 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mfma32f(x[j], qs[4 * i + j], sc);
     }
-  if (partial && hh == 0) {
-    a.part_ml[2 * pr] = M;
-    a.part_ml[2 * pr + 1] = l;
+    const int kk = k0 + 4 * hh - lim;
+    const bool masked = k0 + 31 > klim_lo;  // wave-uniform
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      if (masked && kk + 8 * (r >> 2) + (r & 3) > 0) sc[r] = -INFINITY;
+      tmax = fmaxf(tmax, sc[r]);
+    }
+    tmax = fmaxf(tmax, shfl_xor_f(tmax, 32)) * a.scale_log2;
+    const float mn = fmaxf(m, tmax);
+    const float alpha = mn == m ? 1.0f : fast_exp2(m - mn);
+    const float nm = mn == -INFINITY ? 0.0f : -mn;  // no finite score yet: weights 0
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sc[r] = fast_exp2(fmaf(sc[r], a.scale_log2, nm));
+      l += sc[r];
+    }
+#pragma unroll
+    for (int dt = 0; dt < C::NDT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+    if (!masked) {  // MFMA r sums the keys of register r of both halves
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const char* v = vl + (8 * (r >> 2) + 4 * hh + (r & 3)) * C::VP32 + 4 * c32;
+#pragma unroll
+        for (int dt = 0; dt < C::NDT; ++dt)
+          mfma32f(*reinterpret_cast<const float*>(v + 128 * dt), sc[r], o[dt]);
+      }
+    } else {  // a row's own keys only: 0 times an infinity that it does not see is NaN
+      float* pl = reinterpret_cast<float*>(lds + 2 * C::STAGE32 + wave * C::P32);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) pl[(8 * (r >> 2) + 4 * hh + (r & 3)) * 32 + c32] = sc[r];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int k = 0; k < 32; ++k) {
+        const float p = pl[k * 32 + c32];
+        const bool seen = k0 + k <= lim;
+#pragma unroll
+        for (int dt = 0; dt < C::NDT; ++dt)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(
+                vl + k * C::VP32 + 4 * (32 * dt + 8 * q4 + 4 * hh));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              o[dt][4 * q4 + j] = seen ? fmaf(p, v[j], o[dt][4 * q4 + j]) : o[dt][4 * q4 + j];
+          }
+      }
+    }
+  };
+  ids(t_lo);
+  loads(t_lo);
+  __syncthreads();  // the merge's values have been read
+  for (int t = t_lo; t < n_steps; ++t) {
+    char* base = lds + (t & 1) * C::STAGE32;
+#pragma unroll
+    for (int i = 0; i < C::PASS; ++i) {
+      const int key = lkey + (C::NT / C::CH) * i;
+      st16(base + key * C::KP32 + lbyte, kreg[i]);
+      st16(base + kSKeys * C::KP32 + key * C::VP32 + lbyte, vreg[i]);
+    }
+    __syncthreads();
+    ids(t + 1);
+    loads(t + 1);
+    const int k0 = t * kSKeys + 32 * kg;
+    if (mine && k0 < k_hi && k0 <= klim_hi) again_step(t);  // wave-uniform
   }
+  full_sum();
+  __syncthreads();  // every wave has read its tiles
+  hand_over();
+  merge_store(mine);
 }
 
 template <int HD, int RG>

@@ -387,3 +387,47 @@ def test_f32_split_minus_infinity_scores(gpu, prior, chunk, keys, fused, product
     # keys in one chain: 2,240 roundings of 2^-24 at random, below 2.9e-6
     assert np.abs(got - ref)[fin].max() <= 7e-6 * np.abs(c.vp).max()
     c.close()
+
+
+@pytest.mark.parametrize("R", [1, 7])
+@pytest.mark.parametrize("prior", [0, 1100])
+def test_f32_split_computes_only_rows_that_are_not_finite_again(gpu, R, prior):
+    # a NaN in one query leaves every other row of its workgroup bit for bit
+    c = PCase(gpu, wl.F32, 2 * R, 2, 64, 16, [prior], [150], seed=R + prior)
+    want = c.run().reshape(c.q.shape)
+    at = [(0, 0), (77, R), (149, 2 * R - 1)]
+    for t, h in at:
+        c.q[t, h, 9] = np.nan
+    got = c.run().reshape(c.q.shape)
+    for t, h in at:
+        assert np.isnan(got[t, h]).all()
+        want[t, h] = got[t, h]
+    assert np.array_equal(got, want, equal_nan=True)
+    c.close()
+
+
+def test_f32_split_values_that_are_not_finite_take_no_longer(gpu):
+    # a NaN that every row sees: the rows again on the f32 MFMA, about the time
+    # of two calls more (120 times a call's when keys were walked one by one)
+    c = PCase(gpu, wl.F32, 14, 2, 64, 16, [0], [2048], seed=9)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+    args = (dev(c.q), dev(c.cu), dev(c.ctx), dev(c.tables))
+
+    def ms():
+        layer, best = c.cache.layer(0), 1e9
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            layer.prefill_attention(*args, max_q_len=2048, max_context_len=2048, scale=c.scale)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    plain = ms()
+    b, o = c.tables[0, 0], 0
+    c.kp[b, o, :, 5] = np.nan
+    c.cache.write_bytes(0, pagedkv.K, c.kp)
+    assert np.isnan(c.run()).all()
+    assert ms() < 12 * plain
+    c.close()
