@@ -4,7 +4,8 @@
 // The f32 MFMA (v_mfma_f32_16x16x4f32) does 64 flops per cycle and SIMD, the
 // bf16 one 1,024.  Every f32 operand here is split into three bf16 values,
 // x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1):
-// 24 significant bits, the f32's own), and a product is the six bf16 products
+// 24 significant bits, the f32's own, of values above 2^-102; below, x2 falls
+// out of bf16's range), and a product is the six bf16 products
 // x0 y0, x0 y1, x1 y0, x0 y2, x1 y1, x2 y0 with f32 accumulation: exact
 // products, and what is left out (x1 y2, x2 y1, x2 y2) is below 2^-25 of the
 // product.  Six bf16 MFMAs take 6/16 of the f32 MFMA's time.  The small
@@ -31,7 +32,13 @@
 // The split of a value beyond bf16's range (|x| > 3.39e38, infinities) leaves
 // NaN in its remainders, so every sum it enters ends as NaN: rows whose sums
 // are not all finite are computed again from the f32 values on the f32 MFMA,
-// and such inputs give what f32 arithmetic gives.
+// and such inputs give what f32 arithmetic gives.  So are rows that small
+// values reach: a query with an element outside [2^-100, 2^64] (other than 0;
+// within, a K element below 2^-102 shifts a score by 2^-56 at most), and rows
+// with an output below kSmallOut that is not 0 (V elements below 2^-102 are
+// off by 2^-126 at most, 2^-46 of any larger output).  What stays: a V column
+// of f32 denormals alone may count as 0, and a weight below 2^-102 of the
+// row's largest has fewer bits, which only a V element above 2^80 shows.
 #include <type_traits>
 
 #include "pkv_prefill_dev.h"
@@ -40,6 +47,11 @@ namespace pkv {
 namespace {
 
 constexpr int kSKeys = kSplitKeys;   // keys per step (2 groups of 32)
+constexpr float kSmallOut = 0x1p-80f;
+constexpr int kQMin = (127 - 100) << 7, kQMax = (127 + 64) << 7;  // bf16 words of 2^-100, 2^64
+
+// |x| in an order-preserving word with 0 last (of finite values).
+__device__ __forceinline__ uint32_t mag_word(float x) { return 2u * __float_as_uint(x) - 1u; }
 
 // RG groups of 32 rows times two key groups: 2 RG waves.
 template <int HD, int RG>
@@ -332,6 +344,23 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   //      rows and ids past the last step are clamped (valid, unused) ----
   loads(t_lo);
   ids(t_lo + 1);
+  // queries out of the range in which small keys are exact enough (from their
+  // first parts; computed while the first rows are on the way)
+  unsigned long long q_far;
+  {
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+    us2 lo = us2{0xffff, 0xffff}, hi = us2{0, 0};
+#pragma unroll
+    for (int ks = 0; ks < C::NKQ; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const us2 w = __builtin_bit_cast(us2, qf[0][ks][i] & 0x7fff7fffu);
+        hi = __builtin_elementwise_max(hi, w);
+        lo = __builtin_elementwise_min(lo, (us2)(w - us2{1, 1}));  // (0 last)
+      }
+    q_far = __builtin_amdgcn_ballot_w64(min(lo[0], lo[1]) < kQMin - 1 || max(hi[0], hi[1]) > kQMax);
+  }
+  __builtin_amdgcn_sched_barrier(0);
   store(t_lo & 1);
   loads(t_lo + 1);
   ids(t_lo + 2);
@@ -349,22 +378,31 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   if (bad_block) atomicOr(a.err, PKV_EBIT_BLOCK);
 
   // ---- rows to compute again: a sum that is not finite (a value whose split
-  //      overflowed, or an infinity or NaN in the inputs), or no weight in key
-  //      group 0, which every row sees (its products all overflowed to -inf) ----
+  //      overflowed, or an infinity or NaN in the inputs); no weight in key
+  //      group 0, which every row sees (its products all overflowed to -inf);
+  //      values too small for the split (or a query too large for such keys) ----
   auto full_sum = [&]() __attribute__((always_inline)) {  // both halves' part of l
     const auto lw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(lw[0]) + __uint_as_float(lw[1]);
   };
   full_sum();
   {
-    float z = l;
+    float z[4] = {l, 0.0f, 0.0f, 0.0f};  // 0 times every sum: NaN if one is not finite
+    uint32_t least = ~0u;
 #pragma unroll
     for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) z = fmaf(o[dt][r], 0.0f, z);
-    const unsigned long long w = __builtin_amdgcn_ballot_w64(
-        roww + c32 < n_rows && (!(fabsf(z) < INFINITY) || (kg == 0 && l == 0.0f)));
-    if (w && lane == 0) atomicOr(&again[rw], (uint32_t)w | (uint32_t)(w >> 32));
+      for (int r = 0; r < 16; ++r) {
+        z[r & 3] = fmaf(o[dt][r], 0.0f, z[r & 3]);
+        least = min(least, mag_word(o[dt][r]));
+      }
+    const float zs = (z[0] + z[1]) + (z[2] + z[3]);
+    const unsigned long long w =
+        __builtin_amdgcn_ballot_w64(!(fabsf(zs) < INFINITY) || (kg == 0 && l == 0.0f) ||
+                                    least < mag_word(l * kSmallOut)) | q_far;
+    const uint32_t left = max(n_rows - roww, 0);  // rows of this wave
+    const uint32_t rows = ((uint32_t)w | (uint32_t)(w >> 32)) & (left < 32u ? (1u << left) - 1u : ~0u);
+    if (rows && lane == 0) atomicOr(&again[rw], rows);
   }
 
   // ---- merge of the two key groups: group 1 hands (m, l, O) over in LDS,
@@ -417,12 +455,15 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
     }
   };
   hand_over();
-  const uint32_t mine = (uint32_t)__builtin_amdgcn_readfirstlane((int)again[rw]);
-  uint32_t any = 0;
+  uint32_t mine = 0, any = 0;
 #pragma unroll
-  for (int i = 0; i < RG; ++i) any |= again[i];
+  for (int i = 0; i < RG; ++i) {
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)again[i]);
+    any |= w;
+    mine = i == rw ? w : mine;
+  }
   merge_store(~mine);
-  if (__builtin_amdgcn_readfirstlane((int)any) == 0) return;  // workgroup-uniform
+  if (any == 0u) return;  // workgroup-uniform
 
   // ---- rows `mine` again on the f32 MFMA, with the same split of rows and
   //      keys over the waves: K and V in LDS as they are (double-buffered),

@@ -431,3 +431,21 @@ def test_f32_split_values_that_are_not_finite_take_no_longer(gpu):
     assert np.isnan(c.run()).all()
     assert ms() < 12 * plain
     c.close()
+
+
+@pytest.mark.parametrize("prior", [0, 1100])
+@pytest.mark.parametrize("q_exp,k_exp,v_exp", [(0, 0, -90), (0, 0, -112), (0, 0, -121), (0, 0, 100),
+                                               (104, -104, 0), (120, -120, 0), (-120, 120, 0), (64, -64, 0),
+                                               (-60, 60, -60)])
+def test_f32_split_values_far_from_one(gpu, prior, q_exp, k_exp, v_exp):
+    # values whose third bf16 part falls out of its range, or whose products
+    # meet others that large: the bound of test_f32_split_products all the same
+    c = PCase(gpu, wl.F32, 14, 2, 64, 16, [prior, 9], [140, 33], seed=7 - v_exp)
+    c.q *= np.float32(2.0) ** q_exp
+    c.kp *= np.float32(2.0) ** k_exp
+    c.vp *= np.float32(2.0) ** v_exp
+    c.cache.write_bytes(0, pagedkv.K, c.kp)
+    c.cache.write_bytes(0, pagedkv.V, c.vp)
+    err = np.abs(c.run() - c.reference())
+    assert err.max() <= 4e-6 * np.abs(c.vp).max(), err.max() / np.abs(c.vp).max()
+    c.close()
