@@ -228,27 +228,33 @@ __global__ void __launch_bounds__(kWavesPerBlock * kWave)
 }
 
 // The merge of launches with many partitions per context (max_parts above
-// kWideMergeParts): one workgroup of kWideWaves waves per query head, each
-// wave taking every kWideWaves-th group of partial rows, summed through LDS.
-// One wave per head walks a 30k-token context's 60 to 120 partial rows in
-// rounds of 8, a chain of memory round trips on a few CUs.  Measured, wide
-// against one wave per head: 3 sequences of 64 heads and 65 to 120 partitions
-// of 512-byte rows 6.0 against 10.8 us (the call 79.3 against 88.2 us); one
-// sequence of 32k tokens, 32 heads and 500 partitions: the call 44.5 against
-// 84.4 us; 4 of 8-16k 43.8 against 50.8.  Up to 32 partitions (four rounds of
-// one wave) the plain merge is as fast: 16 sequences of 4k, 45.6 both.
+// kWideMergeParts): one workgroup of 4 waves per query head, a thread per
+// float of a partial row and residue class of rows, two rounds of up to 32 row
+// loads in flight per thread.  One wave per head walks a 30k-token context's 60
+// to 120 partial rows in rounds of 8, a chain of memory round trips on a few
+// CUs.
+// Each class (the rows that one lane group of decode_merge_kernel takes) is
+// summed in that kernel's order and the classes likewise, so both give the
+// same bits: a row does not depend on the bound or the batch that chose the
+// merge.  Whole calls, wide against one wave per head (head_dim 128, contexts
+// in thousands): 1 sequence of 16-30, 32 heads (up to 470 partitions) 42.4 / 74.0
+// us (39.5 with 8 waves that sum every 8th round each, in an order of their
+// own); 2 of 5-6, 64 heads 21.4 / 28.6; 4 of 8-16, 32 heads 42.8 / 51.2; 8 of
+// 8-16, 32 heads 85.0 / 89.6, 64 heads 92.1 / 95.1.  Up to 32 partitions the
+// plain merge is as fast: 16 sequences of 4, 45.6 both.
 constexpr int kWideMergeParts = 32;
-constexpr int kWideWaves = 8;
+constexpr int kWideWaves = 4;
 
 template <int HD>
 __global__ void __launch_bounds__(kWideWaves * kWave)
     decode_merge_wide_kernel(DecodeKArgs a, int R, int dt) {
-  constexpr int LPR = HD / 4;       // lanes per partial row (16 B each)
-  constexpr int PPI = kWave / LPR;  // partial rows per load instruction
-  constexpr int U = 4;              // row loads in flight per lane
-  __shared__ float red[kWideWaves][HD];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int PPI = kWideWaves * kWave / HD;  // classes: rows p with p % PPI == q
+  constexpr int U = kWave / PPI < 32 ? kWave / PPI : 32;  // rows of a round (<= 64 partitions)
+  static_assert(PPI == kWave / (HD / 4), "the lane groups of decode_merge_kernel");
+  __shared__ float red[kWideWaves * kWave];
   const int lane = threadIdx.x & 63;
+  const int x = threadIdx.x % HD;  // float x of the partial row
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x / HD);  // (HD is a multiple of 64)
   const unsigned qh = blockIdx.x;  // (b, g, h)
   const unsigned pair = qh / (unsigned)a.rq;
   const int h = (int)(qh - pair * (unsigned)a.rq);
@@ -260,52 +266,55 @@ __global__ void __launch_bounds__(kWideWaves * kWave)
   if (n_parts <= 1) return;  // uniform over the workgroup
   const size_t pstride_o = (size_t)R * HD;
   const float* mlb = a.part_ml + (size_t)pair * a.max_parts * kMlFloats + 2 * h;
-  const int q = lane / LPR;  // row group
-  const int c = lane % LPR;  // 16-byte chunk of the row
-  const float* pob = a.part_o + ((size_t)pair * a.max_parts * R + h) * HD + 4 * c;
+  const float* pob = a.part_o + ((size_t)pair * a.max_parts * R + h) * HD + x;
 
+  // a round: rows p0 + q, p0 + q + PPI, .. of the class, and m of partition
+  // p0 + lane
+  struct Round {
+    float o[U], m;
+  };
+  auto load = [&](int p0, Round& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * PPI + q;
+      r.o[u] = p < n_parts ? pob[(size_t)p * pstride_o] : 0.0f;
+    }
+    r.m = p0 + lane < n_parts ? mlb[(size_t)(p0 + lane) * kMlFloats] : -INFINITY;
+  };
+  constexpr int STEP = U * PPI;
+  Round r0, r1;
+  load(0, r0);
   // M and L over all partitions, in every wave
-  float M = -INFINITY;
-  for (int p0 = lane; p0 < n_parts; p0 += kWave) M = fmaxf(M, mlb[(size_t)p0 * kMlFloats]);
+  const float l0 = lane < n_parts ? mlb[(size_t)lane * kMlFloats + 1] : 0.0f;
+  float M = r0.m;
+  for (int p = kWave + lane; p < n_parts; p += kWave) M = fmaxf(M, mlb[(size_t)p * kMlFloats]);
   M = wave_all<true>(M);
-  float L = 0.0f;
-  for (int p0 = lane; p0 < n_parts; p0 += kWave) {
-    const float* e = mlb + (size_t)p0 * kMlFloats;
+  float L = lane < n_parts ? fast_exp2(r0.m - M) * l0 : 0.0f;
+  for (int p = kWave + lane; p < n_parts; p += kWave) {
+    const float* e = mlb + (size_t)p * kMlFloats;
     L += fast_exp2(e[0] - M) * e[1];
   }
   L = wave_all<false>(L);
 
-  f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int p0 = wave * PPI * U; p0 < n_parts; p0 += kWideWaves * PPI * U) {
-    f32x4 ov[U];
-    float mv[U];
+  float acc = 0.0f;
+  auto add = [&](const Round& r) __attribute__((always_inline)) {
+    const float w = fast_exp2(r.m - M);  // 0 for absent rows
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int pp = p0 + u * PPI + q;
-      const bool ok = pp < n_parts;
-      ov[u] = ok ? *reinterpret_cast<const f32x4*>(pob + (size_t)pp * pstride_o)
-                 : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      mv[u] = ok ? mlb[(size_t)pp * kMlFloats] : -INFINITY;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float w = fast_exp2(mv[u] - M);  // 0 for absent rows
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = fmaf(w, ov[u][i], acc[i]);
-    }
+    for (int u = 0; u < U; ++u) acc = fmaf(readlane_f(w, u * PPI + q), r.o[u], acc);
+  };
+  for (int p0 = 0; p0 < n_parts; p0 += 2 * STEP) {  // two rounds in flight
+    if (p0 + STEP < n_parts) load(p0 + STEP, r1);
+    add(r0);
+    if (p0 + STEP >= n_parts) break;
+    if (p0 + 2 * STEP < n_parts) load(p0 + 2 * STEP, r0);
+    add(r1);
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (LPR <= 16) acc[i] = with_lane_xor16<false>(acc[i]);
-    if constexpr (LPR <= 32) acc[i] = with_lane_xor32<false>(acc[i]);
-  }
-  if (lane < LPR) *reinterpret_cast<f32x4*>(&red[wave][4 * c]) = acc;
+  red[threadIdx.x] = acc;
   __syncthreads();
-  const int x = threadIdx.x;  // float x of the partial row
-  if (x >= HD) return;
-  float v = 0.0f;
-#pragma unroll
-  for (int w = 0; w < kWideWaves; ++w) v += red[w][x];
+  if (threadIdx.x >= HD) return;
+  float v = red[x];
+  if constexpr (PPI >= 2) v += red[HD + x];
+  if constexpr (PPI >= 4) v += red[2 * HD + x] + red[3 * HD + x];
   v *= 1.0f / L;
   // float 4 c + i of a partial row is element (c % CH) EPL + 4 (c / CH) + i
   const int epl = dt == PKV_F32 ? 4 : 8;

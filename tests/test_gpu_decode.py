@@ -582,3 +582,39 @@ def test_merge_of_many_partitions(gpu, hd, R, dt, out, longest):
     tol = {wl.F32: 0.0, wl.F16: 2.0 ** -11, wl.BF16: 2.0 ** -8}[dt] if out else 0.0
     assert (np.abs(got - ref) <= ATOL + (RTOL + tol) * np.abs(ref)).all()
     c.close()
+
+
+@pytest.mark.parametrize("hd,R,dt", [(64, 4, wl.F16), (128, 20, wl.BF16), (64, 17, wl.F32)])
+@pytest.mark.parametrize("batch", [32, 33])
+def test_merge_of_many_partitions_by_pairs(gpu, hd, R, dt, batch):
+    # 64 (sequence, kv head) pairs are the most that a workgroup per head
+    # merges; ratios above 16 take a second slice of heads.  One context of 35
+    # partitions, the others of 0 to 3 under the same bound
+    ctx = [35000, 0, 1023, 1024, 2100] + [int(x) for x in wl.randint(batch, batch - 5, 0, 3000)]
+    c = Case(gpu, dt, 2 * R, 2, hd, 16, ctx, seed=batch + R, pool_factor=1.0)
+    _close(c.run(), c.reference()[0], f"batch={batch} R={R}")
+    c.close()
+
+
+@pytest.mark.parametrize("R", [4, 20])
+def test_merge_of_many_partitions_positions_bound(gpu, R):
+    # the wide merge lays its partitions out over the bounded lengths
+    ctx = [4500, 2300, 4400, 100, 3000, 2200]
+    pos = [4500, 40, 2111, 63, 0, 5000]
+    c = Case(gpu, wl.BF16, 2 * R, 2, 128, 16, ctx, seed=R, fused=True)
+    got = c.run(max_context_len=4501, positions=pos)
+    _close(got, c.reference(pos)[0], f"positions bound, R={R}")
+    c.close()
+
+
+@pytest.mark.parametrize("dt,hd,R", [(wl.BF16, 128, 4), (wl.F16, 64, 8), (wl.F32, 256, 1),
+                                     (wl.F32, 64, 7), (wl.BF16, 128, 20)])
+def test_rows_do_not_depend_on_the_bound(gpu, dt, hd, R):
+    # 64-token partitions: up to 32 of them under the bound one wave per head
+    # merges, above a workgroup per head; the bits are the same
+    ctx = [2047, 1500, 64, 100, 1999]
+    c = Case(gpu, dt, 2 * R, 2, hd, 16, ctx, seed=hd + R)
+    tight = c.run()
+    for bound in (2049, 3000, 5000):
+        assert np.array_equal(c.run(max_context_len=bound), tight), bound
+    c.close()
