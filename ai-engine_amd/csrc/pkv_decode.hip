@@ -242,7 +242,17 @@ __global__ void __launch_bounds__(kWavesPerBlock * kWave)
 // own); 2 of 5-6, 64 heads 21.4 / 28.6; 4 of 8-16, 32 heads 42.8 / 51.2; 8 of
 // 8-16, 32 heads 85.0 / 89.6, 64 heads 92.1 / 95.1.  Up to 32 partitions the
 // plain merge is as fast: 16 sequences of 4, 45.6 both.
+// More than 64 (sequence, kv head) pairs are cut until there are 2,048
+// partitions, about 32 each, so contexts up to 32k have no more, and of 33-40
+// the merge is lost in the reads (16 sequences 421 / 423, 64 of them 1,521 /
+// 1,522).  What a call with a bound far above its contexts gets there is a
+// launch of 4 times the waves: 256 sequences of 0.5-4 under 40k, 64 heads 455 /
+// 447, 32 heads 438 / 434; 64 of them 131 / 128 and 121 / 120.  Rows of 64
+// floats, a wave per class, gain even so: 256 sequences, 32 heads 242 / 247, 64
+// of them 69.3 / 70.1.  So wide for up to 64 pairs (8 sequences of 0.5-4 under
+// 40k, 64 heads 73.6 / 73.1, 32 heads 61.8 / 61.4) or rows of 64.
 constexpr int kWideMergeParts = 32;
+constexpr size_t kWideMergePairs = 64;
 constexpr int kWideWaves = 4;
 
 template <int HD>
@@ -499,7 +509,8 @@ hipError_t launch_decode_merge(const pkv_pool* p, const DecodeKArgs& k, hipStrea
   if (k.max_parts <= 1) return hipSuccess;
   const int R = group_width(k.rtot);
   const size_t pairs = (size_t)k.batch * k.kvh;
-  if (k.max_parts > kWideMergeParts && grid_fits((long long)pairs * k.rq, kWideWaves * kWave)) {
+  if (k.max_parts > kWideMergeParts && (pairs <= kWideMergePairs || p->head_dim == 64) &&
+      grid_fits((long long)pairs * k.rq, kWideWaves * kWave)) {
     const unsigned grid = (unsigned)(pairs * k.rq);
     switch (p->head_dim) {
       case 64: decode_merge_wide_kernel<64><<<grid, kWideWaves * kWave, 0, stream>>>(k, R, p->dtype); break;
