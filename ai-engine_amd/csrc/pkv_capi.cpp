@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "alloc_retry.h"
 #include "compact_plan.h"
 #include "pkv_internal.h"
 
@@ -64,6 +65,27 @@ struct DeviceGuard {
     (p)->last_error.clear();                                            \
   } while (0)
 
+// hipMalloc on the current device, without the scratch that sampling keeps
+// (up to 512 MiB of free memory) when memory runs out.  stream: the call's,
+// which may be in capture (then nothing is waited for).
+hipError_t device_malloc(void** out, size_t bytes, int device, hipStream_t stream = nullptr) {
+  return pkv::alloc_trimming(
+      hipErrorOutOfMemory,
+      [&]() {
+        const hipError_t e = hipMalloc(out, bytes);
+        if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+        return e;
+      },
+      [&]() { pkv::scratch_trim(device); },
+      [&]() {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const bool ok = hipStreamIsCapturing(stream, &cap) == hipSuccess;
+        if (!ok) (void)hipGetLastError();
+        return ok && cap == hipStreamCaptureStatusNone;
+      },
+      []() { (void)hipDeviceSynchronize(); });
+}
+
 int check_layer(pkv_pool* p, int layer) {
   if (layer < 0 || layer >= p->n_layers)
     return fail(p, PKV_ERR_INVALID, "layer %d out of range [0, %d)", layer,
@@ -93,13 +115,13 @@ int release_retired(pkv_pool* p) {
 // size: a growth that would keep more synchronises and frees them first.
 // Each growth is at least 1.25x, so this keeps at most one old buffer
 // (< 0.8x of the live one) and synchronises at every second growth at most.
-int ensure_workspace(pkv_pool* p, size_t need) {
+int ensure_workspace(pkv_pool* p, size_t need, void* stream = nullptr) {
   if (p->ws && p->ws_bytes >= need) return PKV_OK;
   const size_t bytes = need + need / 4;  // headroom against regrowth
   if (p->ws && p->ws_retired_bytes + p->ws_bytes > bytes)
     if (int rc = release_retired(p)) return rc;
   void* ws = nullptr;
-  hipError_t e = hipMalloc(&ws, bytes);
+  hipError_t e = device_malloc(&ws, bytes, p->device, static_cast<hipStream_t>(stream));
   if (e != hipSuccess)
     return fail(p, PKV_ERR_OOM, "workspace hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   if (p->ws) {
@@ -176,19 +198,13 @@ int pkv_pool_create(pkv_pool** out, int n_layers, int num_blocks,
     return fail(nullptr, PKV_ERR_HIP, "hipSetDevice(%d) failed", device);
   }
   void* base = nullptr;
-  hipError_t e = hipMalloc(&base, total);
-  if (e == hipErrorOutOfMemory) {  // without the scratch that sampling keeps
-    (void)hipGetLastError();
-    (void)hipDeviceSynchronize();
-    pkv::scratch_trim(device);
-    e = hipMalloc(&base, total);
-  }
+  hipError_t e = device_malloc(&base, total, device);
   if (e != hipSuccess) {
     delete p;
     return fail(nullptr, PKV_ERR_OOM, "pool hipMalloc(%zu bytes): %s", total, hipGetErrorString(e));
   }
   void* err = nullptr;
-  e = hipMalloc(&err, 256);
+  e = device_malloc(&err, 256, device);
   if (e == hipSuccess) e = hipMemset(base, 0, total);  // Tensor::zeros
   if (e == hipSuccess) e = hipMemset(err, 0, 256);
   if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -205,7 +221,7 @@ int pkv_pool_create(pkv_pool** out, int n_layers, int num_blocks,
   p->plan_bytes = pkv::plan_capacity_bytes(num_blocks);
   void* dplan = nullptr;
   void* hplan = nullptr;
-  e = hipMalloc(&dplan, p->plan_bytes);
+  e = device_malloc(&dplan, p->plan_bytes, device);
   if (e == hipSuccess) e = hipHostMalloc(&hplan, p->plan_bytes, hipHostMallocDefault);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&p->plan_uploaded, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&p->plan_consumed, hipEventDisableTiming);
@@ -638,7 +654,7 @@ static int decode_call(pkv_pool* p, int layer, pkv::DecodeArgs& a, void* stream,
     if (e != hipSuccess) return hip_fail(p, e, "decode_noalloc launch");
     return PKV_OK;
   }
-  if (int rc = ensure_workspace(p, need)) return rc;
+  if (int rc = ensure_workspace(p, need, stream)) return rc;
   hipEvent_t eb = nullptr, ee = nullptr;
   if (int rc = profile_slot(p, &eb, &ee)) return rc;
   hipError_t e = pkv::launch_decode(p, layer, a, p->ws,
@@ -758,7 +774,7 @@ int prefill_call(pkv_pool* p, int layer, const void* q, void* out, int out_dtype
     size_t need = 0;
     pkv::prefill_plan(p, n_seqs, n_head, max_q_len, max_context_len, &pk, &mp, &need);
     if (need)
-      if (int rc = ensure_workspace(p, need)) return rc;
+      if (int rc = ensure_workspace(p, need, stream)) return rc;
   }
   pkv::PrefillArgs a{q, out, out_dtype, cu_q_lens, context_lens, block_tables,
                      max_blocks_per_seq, n_seqs, max_q_len, max_context_len, n_head, scale,
@@ -897,7 +913,7 @@ int pkv_mixed_attention(pkv_pool* p, int layer, const pkv_prefill_batch* pb,
   DeviceGuard dg(p->device);
   size_t dbytes = 0, pbytes = 0;
   mixed_ws(p, n_head, *pb, *db, &dbytes, &pbytes);
-  if (int rc = ensure_workspace(p, dbytes + pbytes)) return rc;
+  if (int rc = ensure_workspace(p, dbytes + pbytes, stream)) return rc;
   pkv::PrefillArgs pa{pb->q, pb->out, pb->out_dtype, pb->cu_q_lens, pb->context_lens,
                       pb->block_tables, pb->max_blocks_per_seq, pb->n_seqs, pb->max_q_len,
                       pb->max_context_len, n_head, scale, pb->k_new, pb->v_new};
@@ -959,9 +975,9 @@ int pkv_rope_create(pkv_rope** out, int rope_dim, float freq_base, int max_seq, 
   r->device = device;
   DeviceGuard dg(device);
   void *dc = nullptr, *ds = nullptr, *de = nullptr;
-  hipError_t e = hipMalloc(&dc, n * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&ds, n * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&de, 256);
+  hipError_t e = device_malloc(&dc, n * sizeof(float), device);
+  if (e == hipSuccess) e = device_malloc(&ds, n * sizeof(float), device);
+  if (e == hipSuccess) e = device_malloc(&de, 256, device);
   if (e == hipSuccess) e = hipMemcpy(dc, c.data(), n * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(ds, s.data(), n * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(de, 0, 256);

@@ -3561,6 +3561,7 @@ hipError_t scratch_alloc(void** p, size_t bytes, hipStream_t stream) {
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone)
     if (hipMemPool_t pool = scratch_pool(stream)) {
       if (hipMallocFromPoolAsync(p, bytes, pool, stream) == hipSuccess) return hipSuccess;
+      (void)hipMemPoolTrimTo(pool, 0);  // what it keeps is too small and in the way
     }
   (void)hipGetLastError();
   return hipMallocAsync(p, bytes, stream);

@@ -531,7 +531,8 @@ int pkv_sample_exact_routes(const void* logits, int dtype, long long row_stride,
 int pkv_sample_expf(const float* in, float* out, long long n, void* stream);
 /* Gives back the free scratch that pkv_sample and pkv_sample_exact keep on the
  * calling thread's current device (waits for the device; the next call
- * allocates again).  pkv_pool_create does the same when memory runs out. */
+ * allocates again).  Every device allocation of this library does the same
+ * when memory runs out (without the wait while its stream is captured). */
 int pkv_sample_trim(void);
 /* StdRng::seed_from_u64(seed).gen::<f32>() (sample.rs:41-42; host only). */
 float pkv_sample_draw(uint64_t seed);

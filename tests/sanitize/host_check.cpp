@@ -11,6 +11,9 @@
 //     source s held, every other block keeps its bytes), no block is in two
 //     chains (chains run concurrently on the GPU), plan size within the
 //     capacity bound, bad inputs refused;
+//   * allocation with the kept scratch given back (alloc_retry.h): what is
+//     called in which order, for memory that the trim or only the wait frees,
+//     for none, in capture, and for other errors;
 //   * scheduler: block accounting (free + blocks held by live sequences ==
 //     pool), plan arrays within the pool, one token per producing row.
 // Exit status 0 when every check passed.
@@ -24,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "../../ai-engine_amd/csrc/alloc_retry.h"
 #include "../../ai-engine_amd/csrc/compact_plan.h"
 #include "../../include/pagedkv.h"
 
@@ -54,6 +58,45 @@ struct Rng {  // splitmix64
   }
   int below(int n) { return n > 0 ? (int)(next() % (uint64_t)n) : 0; }
 };
+
+// ---- allocation with the kept scratch given back ---------------------------
+void check_alloc_retry() {
+  constexpr int kOk = 0, kOther = 1, kOom = 2;
+  struct Case {
+    int free, kept, in_use, need;  // in_use: kept bytes that queued work still uses
+    bool may_sync;
+    int other;  // the first call fails otherwise
+    int want;
+    const char* calls;
+  };
+  const Case cases[] = {
+      {10, 5, 0, 10, true, 0, kOk, "a"},      {8, 5, 0, 10, true, 0, kOk, "ata"},
+      {8, 5, 5, 10, true, 0, kOk, "atasta"},  {8, 5, 5, 10, false, 0, kOom, "ata"},
+      {8, 1, 0, 10, true, 0, kOom, "atasta"}, {10, 5, 0, 10, true, 1, kOther, "a"},
+  };
+  for (const Case& k : cases) {
+    Case c = k;
+    std::string calls;
+    const int got = pkv::alloc_trimming(
+        kOom,
+        [&]() {
+          calls += 'a';
+          return c.other ? kOther : c.free >= c.need ? kOk : kOom;
+        },
+        [&]() {
+          calls += 't';
+          c.free += c.kept - c.in_use;
+          c.kept = c.in_use;
+        },
+        [&]() { return c.may_sync; },
+        [&]() {
+          calls += 's';
+          c.in_use = 0;
+        });
+    CHECK(got == k.want && calls == k.calls, "alloc_trimming: %d, calls %s instead of %d, %s", got,
+          calls.c_str(), k.want, k.calls);
+  }
+}
 
 // ---- allocator against a model -------------------------------------------
 void check_allocator(uint64_t seed) {
@@ -323,6 +366,7 @@ void check_sched(uint64_t seed) {
 
 int main(int argc, char** argv) {
   const int rounds = argc > 1 ? std::atoi(argv[1]) : 200;
+  check_alloc_retry();
   for (int i = 0; i < rounds; ++i) {
     check_allocator(1000 + i);
     check_planner(2000 + i);

@@ -152,3 +152,18 @@ def test_pool_create_validates_before_touching_device():
         assert b"pool shape" in L.pkv_last_error(None)
     assert L.pkv_pool_destroy(None) == 0
     assert L.pkv_append(None, 0, None, None, None, 1, None) == _lib.PKV_ERR_INVALID
+
+
+def test_every_device_allocation_can_give_the_kept_scratch_back():
+    # one hipMalloc in the library's sources: the one that retries without the
+    # scratch that sampling keeps (its order of steps: tests/sanitize)
+    import glob
+    import os
+    import re
+    csrc = os.path.join(os.path.dirname(_lib.__file__), "..", "csrc")
+    found = []
+    for path in sorted(glob.glob(os.path.join(csrc, "*"))):
+        if path.endswith((".cpp", ".hip", ".h")):
+            src = re.sub(r'//.*|"[^"\n]*"', "", open(path).read())  # comments, messages
+            found += [os.path.basename(path)] * len(re.findall(r"\bhipMalloc\s*\(", src))
+    assert found == ["pkv_capi.cpp"], found
