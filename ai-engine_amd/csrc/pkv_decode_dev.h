@@ -59,7 +59,11 @@ struct DCfg {
   // below GQA 8.  At GQA 8 with bf16 rows of 128, tiles of 48 / 32 / 16 tokens
   // (two waves per SIMD; fewer registers with 16) ran 3 sequences of 16-30k
   // tokens in 79.5 / 74.3 / 72.9 us, 4 of 8-16k in 54.9 / 51.7 / 47.8, 32 of
-  // 1-4k in 84.8 / 82.7 / 82.6 and 128 of 0.5-4k in 218 / 215.4 / 216: 16.
+  // 1-4k in 84.8 / 82.7 / 82.6 and 128 of 0.5-4k in 218 / 215.4 / 216; 64 of
+  // 0.5-4k 147.5 / 144.2 / 144.8, 256 of 0.5-2.5k 280 / 276 / 282.5: 16.  f16
+  // (fewer registers) gains less from 16 and loses more: 4 of 8-16k 52.7
+  // against 50.7 with 16, but 128 of 0.5-4k 205 against 213.5 and 256 of
+  // 0.5-2.5k 280 against 287-293, so it keeps 32.
   static constexpr int NSTMAX =
       (R >= 16  ? 16
        : !ROPE  ? 32

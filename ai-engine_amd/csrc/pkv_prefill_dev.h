@@ -113,10 +113,7 @@ PrefillKArgs prefill_kargs(const pkv_pool* p, int layer, const PrefillArgs& a, c
 hipError_t launch_prefill_merge(const pkv_pool* p, const PrefillKArgs& k, hipStream_t stream);
 // f32 pools of head_dim 64 (pkv_prefill_split.hip): rows per workgroup and
 // keys per step, and the launch.
-#ifndef PKV_SPLIT_ROWS
-#define PKV_SPLIT_ROWS 128
-#endif
-constexpr int kSplitRows = PKV_SPLIT_ROWS, kSplitKeys = 64;
+constexpr int kSplitRows = 128, kSplitKeys = 64;
 hipError_t launch_prefill_split(const PrefillKArgs& k, hipStream_t s);
 
 // Workgroups of the launch; sets the row-block count and the XCD affinity

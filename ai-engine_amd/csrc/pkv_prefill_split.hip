@@ -22,7 +22,7 @@
 // LDS at the end.  K and V are split once per workgroup where they are stored
 // to LDS (three bf16 planes each), Q once in registers, the weights per lane.
 // Against the f32 MFMA kernel (64 rows per workgroup), whole calls on one box:
-// the 6 prompts 60.7 -> 38.8 us, one prompt of 775 tokens 43.8 -> 36.1, of
+// the 6 prompts 59.7 -> 36.7 us, one prompt of 775 tokens 43.8 -> 36.1, of
 // 2,048 121.7 -> 96.3, 6 of 256 27.7 -> 17.9, 6 of 775 114.8 -> 57.4.  A step
 // takes 2.7 us (48 MFMAs a wave, 1,536 cycles; 280 VALU instructions): running
 // the key groups one phase apart, matrix against vector work with a barrier
@@ -39,6 +39,10 @@
 // off by 2^-126 at most, 2^-46 of any larger output).  What stays: a V column
 // of f32 denormals alone may count as 0, and a weight below 2^-102 of the
 // row's largest has fewer bits, which only a V element above 2^80 shows.
+//
+// head_dim 128 and 256 stay on the f32 MFMA (pkv_prefill.hip): two stages of
+// the six planes would take 204 and 396 KB of LDS; a step of 32 keys (102 KB at
+// 128), which leaves one key group, has not been built.
 #include <type_traits>
 
 #include "pkv_prefill_dev.h"
@@ -46,6 +50,8 @@
 namespace pkv {
 namespace {
 
+constexpr int HD = 64;               // head_dim
+constexpr int RG = kSplitRows / 32;  // groups of 32 rows; times two key groups: 2 RG waves
 constexpr int kSKeys = kSplitKeys;   // keys per step (2 groups of 32)
 constexpr float kSmallOut = 0x1p-80f;
 constexpr int kQMin = (127 - 100) << 7, kQMax = (127 + 64) << 7;  // bf16 words of 2^-100, 2^64
@@ -53,10 +59,8 @@ constexpr int kQMin = (127 - 100) << 7, kQMax = (127 + 64) << 7;  // bf16 words 
 // |x| in an order-preserving word with 0 last (of finite values).
 __device__ __forceinline__ uint32_t mag_word(float x) { return 2u * __float_as_uint(x) - 1u; }
 
-// RG groups of 32 rows times two key groups: 2 RG waves.
-template <int HD, int RG>
 struct SCfg {
-  static constexpr int ROWS = 32 * RG;
+  static constexpr int ROWS = kSplitRows;
   static constexpr int NT = 128 * RG;           // threads
   static constexpr int RB = HD * 4;             // row bytes in the pool
   static constexpr int CH = RB / 16;            // 16-byte chunks per row
@@ -103,9 +107,9 @@ __device__ __forceinline__ void mfma32f(float a, float b, f32x16& acc) {
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
 }
 
-template <int HD, int RG, bool FUSED>
-__global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a) {
-  using C = SCfg<HD, RG>;
+template <bool FUSED>
+__global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a) {
+  using C = SCfg;
   __shared__ __attribute__((aligned(16))) char lds[2 * C::STAGE];
   __shared__ uint32_t again[RG];  // rows to compute again in f32, a bit each
 
@@ -578,9 +582,11 @@ __global__ void __launch_bounds__(128 * RG) prefill_split_kernel(PrefillKArgs a)
   merge_store(mine);
 }
 
-template <int HD, int RG>
-hipError_t split_launch(PrefillKArgs k, hipStream_t s) {
-  using C = SCfg<HD, RG>;
+}  // namespace
+
+hipError_t launch_prefill_split(const PrefillKArgs& k0, hipStream_t s) {
+  using C = SCfg;
+  PrefillKArgs k = k0;
   k.row_blocks = (int)(((long long)k.max_q_len * k.rq + C::ROWS - 1) / C::ROWS);
   const long long grid = (long long)k.n_seqs * k.kvh * k.row_blocks * k.max_parts;
   if (grid <= 0) return hipSuccess;
@@ -590,16 +596,10 @@ hipError_t split_launch(PrefillKArgs k, hipStream_t s) {
   // XCDs idle (6 prompts x 2 kv heads: 12 pairs on 8 XCDs).
   k.per_xcd = 0;
   if (k.k_new)
-    prefill_split_kernel<HD, RG, true><<<(unsigned)grid, C::NT, 0, s>>>(k);
+    prefill_split_kernel<true><<<(unsigned)grid, C::NT, 0, s>>>(k);
   else
-    prefill_split_kernel<HD, RG, false><<<(unsigned)grid, C::NT, 0, s>>>(k);
+    prefill_split_kernel<false><<<(unsigned)grid, C::NT, 0, s>>>(k);
   return hipGetLastError();
-}
-
-}  // namespace
-
-hipError_t launch_prefill_split(const PrefillKArgs& k, hipStream_t s) {
-  return split_launch<64, kSplitRows / 32>(k, s);
 }
 
 }  // namespace pkv

@@ -3516,11 +3516,13 @@ constexpr size_t kExactScratch = 512ull << 20;
 // The calls' scratch comes from a memory pool of this library per device.
 // The device's default pool gives free memory back at every synchronisation,
 // and a program that reads each step's tokens synchronises between calls, so
-// each call mapped its scratch anew (256 MB for 256 rows): 256 bf16 rows of
-// 128,256 took 448 us a call with a synchronisation after each (now 109) and
-// 86 us without, 8 f32 rows 178 us (now 144).  This pool keeps up to kExactScratch free
-// bytes over a synchronisation (scratch_trim returns them); which memory may
-// be reused by which stream is the runtime's stream order, as before.
+// each call mapped its scratch anew (256 MB for 256 rows): with a
+// synchronisation after each, 256 bf16 rows of 128,256 took 581 us a call (now
+// 119; 81 without) and 8 f32 rows 299 us (now 148; 109 without), calls of 40
+// sizes in turn 720 on average (now 493: the runtime keeps some of the sizes).
+// This pool keeps up to kExactScratch free bytes over a synchronisation
+// (scratch_trim returns them); which memory may be reused by which stream is
+// the runtime's stream order, as before.
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mutex;
 hipMemPool_t scratch_pools[kMaxDevices];  // created by a device's first call
