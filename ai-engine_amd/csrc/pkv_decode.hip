@@ -228,44 +228,47 @@ __global__ void __launch_bounds__(kWavesPerBlock * kWave)
 }
 
 // The merge of launches with many partitions per context (max_parts above
-// kWideMergeParts): one workgroup of 4 waves per query head, a thread per
-// float of a partial row and residue class of rows, two rounds of up to 32 row
-// loads in flight per thread.  One wave per head walks a 30k-token context's 60
-// to 120 partial rows in rounds of 8, a chain of memory round trips on a few
-// CUs.
+// kWideMergeParts): 4 waves per query head, a thread per float of a partial row
+// and residue class of rows, two rounds of up to 32 row loads in flight per
+// thread.  One wave per head walks a 30k-token context's 60 to 470 partial rows
+// in rounds of 8, a chain of memory round trips.  A workgroup takes 64 columns,
+// so that a head's rows are read by up to 4 CUs (one alone reads about 47 GB/s).
 // Each class (the rows that one lane group of decode_merge_kernel takes) is
 // summed in that kernel's order and the classes likewise, so both give the
 // same bits: a row does not depend on the bound or the batch that chose the
 // merge.  Whole calls, wide against one wave per head (head_dim 128, contexts
-// in thousands): 1 sequence of 16-30, 32 heads (up to 470 partitions) 42.4 / 74.0
-// us (39.5 with 8 waves that sum every 8th round each, in an order of their
-// own); 2 of 5-6, 64 heads 21.4 / 28.6; 4 of 8-16, 32 heads 42.8 / 51.2; 8 of
-// 8-16, 32 heads 85.0 / 89.6, 64 heads 92.1 / 95.1.  Up to 32 partitions the
-// plain merge is as fast: 16 sequences of 4, 45.6 both.
+// in thousands): 1 sequence of 16-30, 32 heads (up to 470 partitions) 39.1 / 74.0
+// us, 64 heads 44.0 / 78.6; 2 of 5-6, 64 heads 21.0 / 28.6; 4 of 8-16, 32 heads
+// 43.9 / 52.7; 8 of 8-16, 32 heads 88.4 / 92.5, 64 heads 94.9 / 98.1.  Up to 32
+// partitions the plain merge is as fast: 16 sequences of 4, 45.6 both.
 // More than 64 (sequence, kv head) pairs are cut until there are 2,048
 // partitions, about 32 each, so contexts up to 32k have no more, and of 33-40
 // the merge is lost in the reads (16 sequences 421 / 423, 64 of them 1,521 /
 // 1,522).  What a call with a bound far above its contexts gets there is a
-// launch of 4 times the waves: 256 sequences of 0.5-4 under 40k, 64 heads 455 /
-// 447, 32 heads 438 / 434; 64 of them 131 / 128 and 121 / 120.  Rows of 64
-// floats, a wave per class, gain even so: 256 sequences, 32 heads 242 / 247, 64
-// of them 69.3 / 70.1.  So wide for up to 64 pairs (8 sequences of 0.5-4 under
-// 40k, 64 heads 73.6 / 73.1, 32 heads 61.8 / 61.4) or rows of 64.
+// launch of 4 times the waves: 256 sequences of 0.5-4 under 40k, 64 heads 462 /
+// 448, 32 heads 441 / 434; 64 of them 132.4 / 128.5 and 122.3 / 120.  Rows of 64
+// floats lose nothing: 256 sequences, 32 heads 245 / 247, 64 of them 70.0 both.
+// So wide for up to 64 pairs (8 sequences of 0.5-4 under 40k, 64 heads 73.6 /
+// 73.1, 32 heads 63.0 / 62.5) or rows of 64.
 constexpr int kWideMergeParts = 32;
 constexpr size_t kWideMergePairs = 64;
-constexpr int kWideWaves = 4;
 
 template <int HD>
-__global__ void __launch_bounds__(kWideWaves * kWave)
+struct WideMerge {
+  static constexpr int PPI = kWave / (HD / 4);  // classes: rows p with p % PPI == q, a wave each
+  static constexpr int CG = HD / kWave;         // workgroups per head, 64 columns each
+};
+
+template <int HD>
+__global__ void __launch_bounds__(WideMerge<HD>::PPI * kWave)
     decode_merge_wide_kernel(DecodeKArgs a, int R, int dt) {
-  constexpr int PPI = kWideWaves * kWave / HD;  // classes: rows p with p % PPI == q
+  constexpr int PPI = WideMerge<HD>::PPI, CG = WideMerge<HD>::CG;
   constexpr int U = kWave / PPI < 32 ? kWave / PPI : 32;  // rows of a round (<= 64 partitions)
-  static_assert(PPI == kWave / (HD / 4), "the lane groups of decode_merge_kernel");
-  __shared__ float red[kWideWaves * kWave];
+  __shared__ float red[PPI * kWave];
   const int lane = threadIdx.x & 63;
-  const int x = threadIdx.x % HD;  // float x of the partial row
-  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x / HD);  // (HD is a multiple of 64)
-  const unsigned qh = blockIdx.x;  // (b, g, h)
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned qh = blockIdx.x / CG;  // (b, g, h)
+  const int x = (int)(blockIdx.x % CG) * kWave + lane;  // float x of the partial row
   const unsigned pair = qh / (unsigned)a.rq;
   const int h = (int)(qh - pair * (unsigned)a.rq);
   const int b = (int)(pair / (unsigned)a.kvh);
@@ -294,13 +297,26 @@ __global__ void __launch_bounds__(kWideWaves * kWave)
   constexpr int STEP = U * PPI;
   Round r0, r1;
   load(0, r0);
-  // M and L over all partitions, in every wave
-  const float l0 = lane < n_parts ? mlb[(size_t)lane * kMlFloats + 1] : 0.0f;
-  float M = r0.m;
-  for (int p = kWave + lane; p < n_parts; p += kWave) M = fmaxf(M, mlb[(size_t)p * kMlFloats]);
+  // M and L over all partitions, in every wave (lane: partitions lane, lane +
+  // 64, ..), the first 512 in one round trip
+  constexpr int ML = 8;
+  float mm[ML], ll[ML];
+#pragma unroll
+  for (int i = 0; i < ML; ++i) {
+    const int p = i * kWave + lane;
+    const bool ok = p < n_parts;
+    mm[i] = ok ? mlb[(size_t)p * kMlFloats] : -INFINITY;
+    ll[i] = ok ? mlb[(size_t)p * kMlFloats + 1] : 0.0f;
+  }
+  float M = mm[0];
+#pragma unroll
+  for (int i = 1; i < ML; ++i) M = fmaxf(M, mm[i]);
+  for (int p = ML * kWave + lane; p < n_parts; p += kWave) M = fmaxf(M, mlb[(size_t)p * kMlFloats]);
   M = wave_all<true>(M);
-  float L = lane < n_parts ? fast_exp2(r0.m - M) * l0 : 0.0f;
-  for (int p = kWave + lane; p < n_parts; p += kWave) {
+  float L = fast_exp2(mm[0] - M) * ll[0];  // (absent partitions add 0)
+#pragma unroll
+  for (int i = 1; i < ML; ++i) L += fast_exp2(mm[i] - M) * ll[i];
+  for (int p = ML * kWave + lane; p < n_parts; p += kWave) {
     const float* e = mlb + (size_t)p * kMlFloats;
     L += fast_exp2(e[0] - M) * e[1];
   }
@@ -321,10 +337,10 @@ __global__ void __launch_bounds__(kWideWaves * kWave)
   }
   red[threadIdx.x] = acc;
   __syncthreads();
-  if (threadIdx.x >= HD) return;
-  float v = red[x];
-  if constexpr (PPI >= 2) v += red[HD + x];
-  if constexpr (PPI >= 4) v += red[2 * HD + x] + red[3 * HD + x];
+  if (q != 0) return;
+  float v = acc;
+  if constexpr (PPI >= 2) v += red[kWave + lane];
+  if constexpr (PPI >= 4) v += red[2 * kWave + lane] + red[3 * kWave + lane];
   v *= 1.0f / L;
   // float 4 c + i of a partial row is element (c % CH) EPL + 4 (c / CH) + i
   const int epl = dt == PKV_F32 ? 4 : 8;
@@ -337,6 +353,12 @@ __global__ void __launch_bounds__(kWideWaves * kWave)
   else
     reinterpret_cast<uint16_t*>(a.out)[eo] =
         (uint16_t)(dt == PKV_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v));
+}
+
+template <int HD>
+void merge_wide(unsigned heads, const DecodeKArgs& k, int R, int dt, hipStream_t s) {
+  using W = WideMerge<HD>;
+  decode_merge_wide_kernel<HD><<<heads * W::CG, W::PPI * kWave, 0, s>>>(k, R, dt);
 }
 
 // Block sizes below 16 take the kernels with per-lane block ids.
@@ -510,12 +532,12 @@ hipError_t launch_decode_merge(const pkv_pool* p, const DecodeKArgs& k, hipStrea
   const int R = group_width(k.rtot);
   const size_t pairs = (size_t)k.batch * k.kvh;
   if (k.max_parts > kWideMergeParts && (pairs <= kWideMergePairs || p->head_dim == 64) &&
-      grid_fits((long long)pairs * k.rq, kWideWaves * kWave)) {
-    const unsigned grid = (unsigned)(pairs * k.rq);
+      grid_fits((long long)pairs * k.rq, 4 * kWave)) {  // 4 waves per head
+    const unsigned heads = (unsigned)(pairs * k.rq);
     switch (p->head_dim) {
-      case 64: decode_merge_wide_kernel<64><<<grid, kWideWaves * kWave, 0, stream>>>(k, R, p->dtype); break;
-      case 128: decode_merge_wide_kernel<128><<<grid, kWideWaves * kWave, 0, stream>>>(k, R, p->dtype); break;
-      default: decode_merge_wide_kernel<256><<<grid, kWideWaves * kWave, 0, stream>>>(k, R, p->dtype); break;
+      case 64: merge_wide<64>(heads, k, R, p->dtype, stream); break;
+      case 128: merge_wide<128>(heads, k, R, p->dtype, stream); break;
+      default: merge_wide<256>(heads, k, R, p->dtype, stream); break;
     }
     return hipGetLastError();
   }
