@@ -54,10 +54,7 @@ constexpr int HD = 64;               // head_dim
 constexpr int RG = kSplitRows / 32;  // groups of 32 rows; times two key groups: 2 RG waves
 constexpr int kSKeys = kSplitKeys;   // keys per step (2 groups of 32)
 constexpr float kSmallOut = 0x1p-80f;
-constexpr int kQMin = (127 - 100) << 7, kQMax = (127 + 64) << 7;  // bf16 words of 2^-100, 2^64
-
-// |x| in an order-preserving word with 0 last (of finite values).
-__device__ __forceinline__ uint32_t mag_word(float x) { return 2u * __float_as_uint(x) - 1u; }
+constexpr float kQMin = 0x1p-100f, kQMax = 0x1p64f;
 
 struct SCfg {
   static constexpr int ROWS = kSplitRows;
@@ -213,6 +210,7 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   ids(t_lo);
   // ---- this wave's rows of Q (B operand), three planes ----
   u32x4 qf[3][C::NKQ];
+  float q_lo = INFINITY, q_hi = 0.0f;  // extremes of |q| of this wave's half of the steps
   {
     const char* qrow = a.q + ((size_t)(q0 + rc / R) * H + g * R + rc % R) * C::RB;
 #pragma unroll
@@ -221,6 +219,14 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
       const u32x4 x0 = ld16(qrow + 64 * ks + 32 * hh), x1 = ld16(qrow + 64 * ks + 32 * hh + 16);
       split4(x0, lo);
       split4(x1, hi);
+      if ((ks & 1) == kg) {  // (both key groups hold these rows)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float y0 = fabsf(__uint_as_float(x0[i])), y1 = fabsf(__uint_as_float(x1[i]));
+          q_lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(q_lo, y0), y1);
+          q_hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(q_hi, y0), y1);
+        }
+      }
 #pragma unroll
       for (int q = 0; q < 3; ++q) qf[q][ks] = u32x4{lo[q].x, lo[q].y, hi[q].x, hi[q].y};
     }
@@ -348,23 +354,6 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   //      rows and ids past the last step are clamped (valid, unused) ----
   loads(t_lo);
   ids(t_lo + 1);
-  // queries out of the range in which small keys are exact enough (from their
-  // first parts; computed while the first rows are on the way)
-  unsigned long long q_far;
-  {
-    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-    us2 lo = us2{0xffff, 0xffff}, hi = us2{0, 0};
-#pragma unroll
-    for (int ks = 0; ks < C::NKQ; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const us2 w = __builtin_bit_cast(us2, qf[0][ks][i] & 0x7fff7fffu);
-        hi = __builtin_elementwise_max(hi, w);
-        lo = __builtin_elementwise_min(lo, (us2)(w - us2{1, 1}));  // (0 last)
-      }
-    q_far = __builtin_amdgcn_ballot_w64(min(lo[0], lo[1]) < kQMin - 1 || max(hi[0], hi[1]) > kQMax);
-  }
-  __builtin_amdgcn_sched_barrier(0);
   store(t_lo & 1);
   loads(t_lo + 1);
   ids(t_lo + 2);
@@ -381,32 +370,32 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   }
   if (bad_block) atomicOr(a.err, PKV_EBIT_BLOCK);
 
-  // ---- rows to compute again: a sum that is not finite (a value whose split
-  //      overflowed, or an infinity or NaN in the inputs); no weight in key
-  //      group 0, which every row sees (its products all overflowed to -inf);
-  //      values too small for the split (or a query too large for such keys) ----
   auto full_sum = [&]() __attribute__((always_inline)) {  // both halves' part of l
     const auto lw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(lw[0]) + __uint_as_float(lw[1]);
   };
   full_sum();
-  {
-    float z[4] = {l, 0.0f, 0.0f, 0.0f};  // 0 times every sum: NaN if one is not finite
-    uint32_t least = ~0u;
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        z[r & 3] = fmaf(o[dt][r], 0.0f, z[r & 3]);
-        least = min(least, mag_word(o[dt][r]));
-      }
-    const float zs = (z[0] + z[1]) + (z[2] + z[3]);
-    const unsigned long long w =
-        __builtin_amdgcn_ballot_w64(!(fabsf(zs) < INFINITY) || (kg == 0 && l == 0.0f) ||
-                                    least < mag_word(l * kSmallOut)) | q_far;
+  // rows to compute again, by a lane mask of this wave
+  auto mark = [&](unsigned long long lanes) __attribute__((always_inline)) {
     const uint32_t left = max(n_rows - roww, 0);  // rows of this wave
-    const uint32_t rows = ((uint32_t)w | (uint32_t)(w >> 32)) & (left < 32u ? (1u << left) - 1u : ~0u);
+    const uint32_t rows =
+        ((uint32_t)lanes | (uint32_t)(lanes >> 32)) & (left < 32u ? (1u << left) - 1u : ~0u);
     if (rows && lane == 0) atomicOr(&again[rw], rows);
+  };
+  // queries out of the range in which small keys are exact enough; 0 is in it
+  // (looked at again, from the first parts, only where there is one)
+  if (__builtin_amdgcn_ballot_w64(!(q_lo >= kQMin && q_hi <= kQMax))) {  // wave-uniform
+    bool far = false;
+#pragma unroll
+    for (int ks = 0; ks < C::NKQ; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float y = fabsf(e ? bf16hi(qf[0][ks][i]) : bf16lo(qf[0][ks][i]));
+          far |= (y < kQMin && y != 0.0f) || y > kQMax;
+        }
+    mark(__builtin_amdgcn_ballot_w64(far));
   }
 
   // ---- merge of the two key groups: group 1 hands (m, l, O) over in LDS,
@@ -415,6 +404,7 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   static_assert(RG * kXW * 4 <= 2 * C::STAGE, "");
   float* xo = reinterpret_cast<float*>(lds) + rw * kXW;
   const bool partial = nparts > 1;
+  float* const out_rows = partial ? a.part_o : reinterpret_cast<float*>(a.out);
   const size_t item = ((size_t)sg * a.row_blocks + rb) * a.max_parts + part;
   auto hand_over = [&]() __attribute__((always_inline)) {
     if (kg == 1) {
@@ -429,36 +419,70 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
     }
     __syncthreads();
   };
-  auto merge_store = [&](uint32_t rows) __attribute__((always_inline)) {  // bit c32: row roww + c32
-    if (kg == 1) return;
+  // Key group 0 stores the merged rows: all of them, marking those to compute
+  // again, or (`check` false) the marked ones, bit c32 of rows for row roww +
+  // c32.  Marked are rows with an output that is not finite (a value whose
+  // split overflowed, or an infinity or NaN in the inputs), rows without a
+  // weight in key group 0, which every row sees (its products all overflowed
+  // to -inf), and outputs too small for the split that are not 0.
+  auto merge_store = [&](auto check, uint32_t rows) __attribute__((always_inline)) {
+    constexpr bool CHECK = decltype(check)::value;
     const float m1 = xo[C::NDT * 16 * 64 + lane], l1 = xo[C::NDT * 16 * 64 + 64 + lane];
     const float M = fmaxf(m, m1);
     // (m = m1 = -inf: no finite score, sums of 0)
     const float w0 = m == M ? 1.0f : fast_exp2(m - M), w1 = m1 == M ? 1.0f : fast_exp2(m1 - M);
     l = l * w0 + l1 * w1;
     const int r = roww + c32;
-    if (r >= n_rows || !((rows >> c32) & 1u)) return;
+    const bool live = r < n_rows && (CHECK || ((rows >> c32) & 1u));
     const float f0 = partial ? w0 : w0 / l, f1 = partial ? w1 : w1 / l;
     const size_t pr = item * C::ROWS + (r - row0);
-    float* dst = partial ? a.part_o + pr * HD
-                         : reinterpret_cast<float*>(a.out) +
-                               ((size_t)(q0 + r / R) * H + g * R + r % R) * HD;
+    float* dst = out_rows + (partial ? pr : (size_t)(q0 + r / R) * H + g * R + r % R) * HD;
+    auto merged = [&](int dt, int q4) __attribute__((always_inline)) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(xo + ((dt * 4 + q4) * 64 + lane) * 4);
+      f32x4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = o[dt][4 * q4 + j] * f0 + x[j] * f1;
+      return y;
+    };
+    float lo = INFINITY, hi = 0.0f;  // extremes of |y|, NaN if one is NaN
 #pragma unroll
     for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(xo + ((dt * 4 + q4) * 64 + lane) * 4);
-        f32x4 y;
+        const f32x4 y = merged(dt, q4);
+        if (live) *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * q4 + 4 * hh) = y;
+        if constexpr (CHECK) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) y[j] = o[dt][4 * q4 + j] * f0 + x[j] * f1;
-        *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * q4 + 4 * hh) = y;
+          for (int j = 0; j < 4; ++j) {
+            lo = __builtin_elementwise_minimum(lo, fabsf(y[j]));
+            hi = __builtin_elementwise_maximum(hi, fabsf(y[j]));
+          }
+        }
       }
-    if (partial && hh == 0) {
+    if (partial && live && hh == 0) {
       a.part_ml[2 * pr] = M;
       a.part_ml[2 * pr + 1] = l;
     }
+    if constexpr (CHECK) {
+      const float small = partial ? l * kSmallOut : kSmallOut;
+      const bool fine = lo >= small && hi < INFINITY && m != -INFINITY;
+      if (__builtin_amdgcn_ballot_w64(!fine)) {  // wave-uniform: a 0 among them, or worse
+        bool bad = !(hi < INFINITY) || m == -INFINITY;
+#pragma unroll
+        for (int dt = 0; dt < C::NDT; ++dt)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const f32x4 y = merged(dt, q4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bad |= fabsf(y[j]) < small && y[j] != 0.0f;
+          }
+        mark(__builtin_amdgcn_ballot_w64(bad));
+      }
+    }
   };
   hand_over();
+  if (kg == 0 && has_rows) merge_store(std::true_type{}, ~0u);  // wave-uniform
+  __syncthreads();  // the marks are there, and the merge's values have been read
   uint32_t mine = 0, any = 0;
 #pragma unroll
   for (int i = 0; i < RG; ++i) {
@@ -466,7 +490,6 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
     any |= w;
     mine = i == rw ? w : mine;
   }
-  merge_store(~mine);
   if (any == 0u) return;  // workgroup-uniform
 
   // ---- rows `mine` again on the f32 MFMA, with the same split of rows and
@@ -561,7 +584,6 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   };
   ids(t_lo);
   loads(t_lo);
-  __syncthreads();  // the merge's values have been read
   for (int t = t_lo; t < n_steps; ++t) {
     char* base = lds + (t & 1) * C::STAGE32;
 #pragma unroll
@@ -579,7 +601,7 @@ __global__ void __launch_bounds__(SCfg::NT) prefill_split_kernel(PrefillKArgs a)
   full_sum();
   __syncthreads();  // every wave has read its tiles
   hand_over();
-  merge_store(mine);
+  if (kg == 0 && mine) merge_store(std::false_type{}, mine);
 }
 
 }  // namespace
